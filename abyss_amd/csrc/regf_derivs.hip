@@ -12,9 +12,10 @@
 // derivs23: one target per lane; every lane of a wave walks the same j, so
 // the j record (x, v, a, adot, m; 128-byte AoS copy of the state) is read at
 // a wave-uniform address and reaches the lanes through the scalar cache.
-// The j range is split over grid.y so that small target blocks still fill
-// the chip; partial sums are added in split order by a second kernel
-// (bitwise reproducible).
+// The four waves of a workgroup share 64 targets and take a quarter of the
+// workgroup's j range each; the j range is split over grid.y as well, so
+// that small target blocks still fill the chip.  Partial sums are added in a
+// fixed order (bitwise reproducible).
 #include "regf_context.h"
 
 #include <stdio.h>
@@ -42,90 +43,126 @@ __global__ __launch_bounds__(256) void pack_drec_kernel(const double *__restrict
                   st[13 * N + i], 0.0,            0.0,            0.0};
 }
 
-// One split of the j range for 256 targets.  REF: the reference's signs of
-// the projections x.(a_i - a_j)/r2, v.(a_i - a_j)/r2, x.(adot_i - adot_j)/r2
-// in B and C; !REF: x.(a_j - a_i) etc., the exact derivatives of
-// m x/|x|^3 along the relative orbit (x'' = a_j - a_i).
+// One split of the j range for 64 targets.  The terms are the reference's
+// (x, v, da = a_j - a_i, dj = adot_j - adot_i, w = m/r^3, q = 1/r^2, p = -1
+// for REF, whose projections x.(a_i - a_j)/r2, v.(a_i - a_j)/r2 and
+// x.(adot_i - adot_j)/r2 enter B and C, p = 1 for the exact derivatives of
+// m x/|x|^3 along the relative orbit), collected by vector:
+//   A = (x.v) q,  T = (v.v + p x.da) q,  D = p (3 v.da + x.dj) q
+//   a2 = w da - 6 w A v + w (15 A^2 - 3 T) x
+//   a3 = w dj - 9 w A da + 3 w (15 A^2 - 3 T) v + w (A (45 T - 105 A^2) - 3 D) x
+// which is the reference's B = T + A^2, C = D + A (3 B - 4 A^2) inserted into
+// adot2 = w da - 6 A f1 - 3 B f0, adot3 = w dj - 9 A adot2 - 9 B f1 - 3 C f0.
+// Bound by FP64 VALU issue: 81 instructions per pair with one hardware
+// reciprocal root (refined to second order) and no division; the j records
+// cost no vector instruction.  Written term by term (8 divisions and a square
+// root per pair, one wave walking at least 1024 j) a call took 2194 us at
+// N = m = 16384 and 1022 us at N = 40000, m = 1; now 841 and 47 us.
+// A step with a neighbour, the target itself or an r^2 whose r^-3 is zero
+// takes a branch that moves those lanes' terms to the irregular sums (or
+// drops them) and zeroes their factors.
 template <bool REF>
 __global__ __launch_bounds__(256) void derivs23_kernel(const DRec *__restrict__ jr, int n,
                                                        const int *__restrict__ tgt, int nt,
                                                        const double *__restrict__ rnb2,
                                                        int jspan, double *__restrict__ part)
 {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ double s_sum[3][12][64];   // waves 1 to 3 hand their sums to wave 0
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int q = blockIdx.x * 64 + lane;
     const int s = blockIdx.y;
-    const int j0 = s * jspan;
-    const int j1 = min(n, j0 + jspan);
+    // this wave's quarter of the split (empty for the last waves of a short one)
+    const int sub = (jspan + 3) / 4;
+    const int j0 = s * jspan + wave * sub;
+    const int j1 = min(min(n, (s + 1) * jspan), j0 + sub);
     const bool active = q < nt;
     const int i = active ? tgt[q] : 0;
     const DRec ri = jr[i];
-    const double rn = rnb2[i];
-    const double ps = REF ? 1.0 : -1.0;
-    double reg2[3] = {0, 0, 0}, reg3[3] = {0, 0, 0}, irr2[3] = {0, 0, 0}, irr3[3] = {0, 0, 0};
-    for (int j = j0; j < j1; ++j) {
-        const DRec rj = jr[j];   // wave-uniform address
+    const double rn = active ? rnb2[i] : -1.0;
+    double reg[6] = {0, 0, 0, 0, 0, 0}, irr[6] = {0, 0, 0, 0, 0, 0};   // a2, a3
+    // r^-3 of anything above is below the smallest double
+    constexpr double kFar = 1.0e290;
+    auto pair = [&](const DRec &rj) {
         const double x[3] = {rj.x - ri.x, rj.y - ri.y, rj.z - ri.z};
         const double v[3] = {rj.vx - ri.vx, rj.vy - ri.vy, rj.vz - ri.vz};
-        const double da[3] = {ri.ax - rj.ax, ri.ay - rj.ay, ri.az - rj.az};      // a1 - a2
-        const double dj[3] = {ri.jx - rj.jx, ri.jy - rj.jy, ri.jz - rj.jz};      // a1dot - a2dot
-        const double r2 = x[0] * x[0] + x[1] * x[1] + x[2] * x[2];
-        if (r2 == 0.0) continue;   // self (and coincident j)
-        const double vr = v[0] * x[0] + v[1] * x[1] + v[2] * x[2];
-        const double v2 = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
-        const double r3 = r2 * sqrt(r2);
-        const double m_r3 = rj.m / r3;
-        const double inv_r2 = 1.0 / r2;
-        double a21[3], a21dot[3];
-        double rdf = 0, vdf = 0, rdfdot = 0;
+        const double da[3] = {rj.ax - ri.ax, rj.ay - ri.ay, rj.az - ri.az};
+        const double dj[3] = {rj.jx - ri.jx, rj.jy - ri.jy, rj.jz - ri.jz};
+        auto dot = [](const double *a, const double *b) {
+            return fma(a[2], b[2], fma(a[1], b[1], a[0] * b[0]));
+        };
+        const double r2 = dot(x, x);
+        const double xa = dot(x, da), xj = dot(x, dj), va = dot(v, da);
+        double y = __builtin_amdgcn_rsq(r2);
+        const double e = fma(-(r2 * y), y, 1.0);
+        y = fma(y * fma(0.375, e, 0.5), e, y);
+        const double iq = y * y;
+        double w = rj.m * y * iq;
+        const double A = dot(v, x) * iq;
+        const double T = (REF ? dot(v, v) - xa : dot(v, v) + xa) * iq;
+        const double D = (REF ? -fma(3.0, va, xj) : fma(3.0, va, xj)) * iq;
+        const double A2 = A * A;
+        const double wA = w * A;
+        double cv = -6.0 * wA, cd = -9.0 * wA;
+        double cx = w * fma(15.0, A2, -3.0 * T);
+        double cy = w * fma(A, fma(45.0, T, -105.0 * A2), -3.0 * D);
+        const bool near = !(r2 > rn);
+        auto add = [&](double *o) {
+            const double cw = 3.0 * cx;
 #pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            a21[d] = m_r3 * x[d];
-            a21dot[d] = m_r3 * (v[d] - 3 * x[d] * vr * inv_r2);
-            rdf += x[d] * da[d];
-            vdf += v[d] * da[d];
-            rdfdot += x[d] * dj[d];
-        }
-        rdf *= ps * inv_r2;
-        vdf *= ps * inv_r2;
-        rdfdot *= ps * inv_r2;
-        const double A = vr * inv_r2;
-        const double B = v2 * inv_r2 + rdf + A * A;
-        const double C = 3 * vdf + rdfdot + A * (3 * B - 4 * A * A);
-        const bool reg = r2 > rn;
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            const double adot2 = -rj.m * da[d] / r3 - 6 * A * a21dot[d] - 3 * B * a21[d];
-            const double adot3 =
-                -rj.m * dj[d] / r3 - 9 * A * adot2 - 9 * B * a21dot[d] - 3 * C * a21[d];
-            if (reg) {
-                reg2[d] += adot2;
-                reg3[d] += adot3;
-            } else {
-                irr2[d] += adot2;
-                irr3[d] += adot3;
+            for (int d = 0; d < 3; ++d) {
+                o[d] = fma(cx, x[d], fma(cv, v[d], fma(w, da[d], o[d])));
+                o[3 + d] = fma(cy, x[d], fma(cw, v[d], fma(cd, da[d], fma(w, dj[d], o[3 + d]))));
+            }
+        };
+        if (__any(near || !(r2 < kFar))) {
+            const bool none = r2 == 0.0 || !(r2 < kFar);   // self, coincident, out of reach
+            if (none) w = cv = cd = cx = cy = 0.0;
+            if (near) {
+                add(irr);
+                w = cv = cd = cx = cy = 0.0;
             }
         }
+        add(reg);
+    };
+    if (j0 < j1) {
+        DRec rj = jr[j0];   // wave-uniform address
+        for (int j = j0; j < j1; ++j) {
+            const DRec next = jr[min(j + 1, j1 - 1)];
+            pair(rj);
+            rj = next;
+        }
     }
-    if (!active) return;
+    if (wave > 0)
+#pragma unroll
+        for (int c = 0; c < 12; ++c) s_sum[wave - 1][c][lane] = c < 6 ? reg[c] : irr[c - 6];
+    __syncthreads();
+    if (wave > 0 || !active) return;
     double *o = part + ((size_t)s * nt + q) * 12;
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        o[d] = reg2[d];
-        o[3 + d] = reg3[d];
-        o[6 + d] = irr2[d];
-        o[9 + d] = irr3[d];
+    for (int c = 0; c < 12; ++c) {
+        double a = c < 6 ? reg[c] : irr[c - 6];
+        for (int k = 0; k < 3; ++k) a += s_sum[k][c][lane];
+        o[c] = a;
     }
 }
 
-// out[q][c] = sum over splits s (in order) of part[s][q][c].
+// out[e] = sum over the splits of part[s][e]: 16 threads per element take the
+// splits s, s + 16, ... in order, and their sums are added in order.
 __global__ __launch_bounds__(256) void derivs_sum_kernel(const double *__restrict__ part, int S,
                                                          int nt, double *__restrict__ out)
 {
-    const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ double s_sum[16][16];
+    const int k = threadIdx.x >> 4, c = threadIdx.x & 15;
+    const size_t e = (size_t)blockIdx.x * 16 + c;
     const size_t total = (size_t)nt * 12;
-    if (e >= total) return;
     double acc = 0.0;
-    for (int s = 0; s < S; ++s) acc += part[(size_t)s * total + e];
+    if (e < total)
+        for (int s = k; s < S; s += 16) acc += part[(size_t)s * total + e];
+    s_sum[k][c] = acc;
+    __syncthreads();
+    if (k > 0 || e >= total) return;
+    for (int t = 1; t < 16; ++t) acc += s_sum[t][c];
     out[e] = acc;
 }
 
@@ -190,11 +227,11 @@ int abyss_ctx_derivs23(abyss_ctx_t c, int nt, const int *targets, int reference_
             return ABYSS_ERR_TARGET_RANGE;
         }
     if (hipSetDevice(c->device) != hipSuccess) return ABYSS_ERR_HIP;
-    // j splits: ~8 workgroups per CU, each split at least 1024 j
-    const int gx = (nt + 255) / 256;
+    // j splits: 16 workgroups per CU, each split at least 64 j (16 per wave)
+    const int gx = (nt + 63) / 64;
     const int cu = c->cu_count > 0 ? c->cu_count : 256;
-    int S = std::max(1, (cu * 8 + gx - 1) / gx);
-    S = std::min(S, std::max(1, n / 1024));
+    int S = std::max(1, (cu * 16 + gx - 1) / gx);
+    S = std::min(S, std::max(1, n / 64));
     S = std::min(S, 1024);
     const int jspan = (n + S - 1) / S;
     S = (n + jspan - 1) / jspan;
@@ -202,22 +239,25 @@ int abyss_ctx_derivs23(abyss_ctx_t c, int nt, const int *targets, int reference_
     const size_t part_bytes = (size_t)S * nt * 12 * sizeof(double);
     const size_t tgt_bytes = (((size_t)nt * sizeof(int)) + 255) & ~size_t(255);
     const size_t out_bytes = (size_t)nt * 12 * sizeof(double);
-    int rc = ensure_buf(&c->d_drv, &c->drv_bytes, rec_bytes + part_bytes + tgt_bytes + out_bytes,
-                        c->stream);
+    int rc = ensure_buf(&c->d_drv, &c->drv_bytes, rec_bytes + part_bytes + tgt_bytes, c->stream);
     if (rc != ABYSS_OK) return rc;
     if (hipStreamSynchronize(c->stream) != hipSuccess) return ABYSS_ERR_HIP;
     if (out_bytes + tgt_bytes > c->h_drv_bytes) {
         if (c->h_drv) (void)hipHostFree(c->h_drv);
         c->h_drv = nullptr;
         c->h_drv_bytes = 0;
-        if (hipHostMalloc(&c->h_drv, out_bytes + tgt_bytes, hipHostMallocDefault) != hipSuccess)
+        if (hipHostMalloc(&c->h_drv, out_bytes + tgt_bytes,
+                          hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
             return ABYSS_ERR_OUT_OF_MEMORY;
         c->h_drv_bytes = out_bytes + tgt_bytes;
     }
+    void *h_dev = nullptr;
+    if (hipHostGetDevicePointer(&h_dev, c->h_drv, 0) != hipSuccess) return ABYSS_ERR_HIP;
+    // the sums go straight into the mapped block, so no copy follows them
+    double *d_out = reinterpret_cast<double *>(static_cast<char *>(h_dev) + tgt_bytes);
     DRec *d_rec = reinterpret_cast<DRec *>(c->d_drv);
     double *d_part = reinterpret_cast<double *>(c->d_drv + rec_bytes);
     int *d_tgt = reinterpret_cast<int *>(c->d_drv + rec_bytes + part_bytes);
-    double *d_out = reinterpret_cast<double *>(c->d_drv + rec_bytes + part_bytes + tgt_bytes);
     memcpy(c->h_drv, targets, (size_t)nt * sizeof(int));
     if (hipMemcpyAsync(d_tgt, c->h_drv, (size_t)nt * sizeof(int), hipMemcpyHostToDevice,
                        c->stream) != hipSuccess)
@@ -232,13 +272,11 @@ int abyss_ctx_derivs23(abyss_ctx_t c, int nt, const int *targets, int reference_
         hipLaunchKernelGGL(derivs23_kernel<false>, dim3(gx, S), dim3(256), 0, c->stream, d_rec,
                            n, d_tgt, nt, st_r2, jspan, d_part);
     const size_t total = (size_t)nt * 12;
-    hipLaunchKernelGGL(derivs_sum_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
+    hipLaunchKernelGGL(derivs_sum_kernel, dim3((unsigned)((total + 15) / 16)), dim3(256), 0,
                        c->stream, d_part, S, nt, d_out);
     if (hipGetLastError() != hipSuccess) return ABYSS_ERR_HIP;
     double *h_out = reinterpret_cast<double *>(c->h_drv + tgt_bytes);
-    if (hipMemcpyAsync(h_out, d_out, out_bytes, hipMemcpyDeviceToHost, c->stream) != hipSuccess ||
-        hipStreamSynchronize(c->stream) != hipSuccess)
-        return ABYSS_ERR_HIP;
+    if (hipStreamSynchronize(c->stream) != hipSuccess) return ABYSS_ERR_HIP;
     memcpy(out, h_out, out_bytes);
     return ABYSS_OK;
 }
