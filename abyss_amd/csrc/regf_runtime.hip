@@ -306,6 +306,23 @@ Plan plan_for(abyss_ctx_t c, int nt, int n, int prec, int cap, bool forced)
         const int s_long = std::max(1, n / (16 * abyss::kTile));
         if (!tuned && !c->batch_member && (long long)p.grid_x * s_long >= 8LL * cu)
             S = std::min(S, s_long);
+        // few workgroups (a small j-set or a small block): shorter spans,
+        // down to one tile and at most 128 splits, up to 8 workgroups per CU
+        // (4 lanes per target) or 4 (16 lanes, whose five resident
+        // workgroups then start at once).  Not for FP32 terms over 16 lanes,
+        // whose runs of 64 pairs take four tiles: shorter spans would cut
+        // them.  Launch times before -> after, N / targets: 16385 / 4096
+        // refined 148 -> 136 us (S = 13 -> 22) and checked 134 -> 124 us,
+        // 65536 / 1000 checked 104.5 -> 102.8 us and 65536 / 64 checked
+        // 29.2 -> 27.0 us (64 -> 128).  More than 128 splits cost more to
+        // merge than they gain (131072 / 30, 512 splits: 29.3 -> 32.2 us;
+        // 65536 / 64, 256 splits: 29.4 us).
+        const long long few = (jl == 4 ? 8LL : 4LL) * cu;
+        if (!tuned && !c->batch_member && (jl == 4 || (jl == 16 && !mode0)) &&
+            (long long)p.grid_x * S < few) {
+            const long long want = std::min<long long>((few + p.grid_x - 1) / p.grid_x, 128);
+            S = std::max(S, (int)std::min<long long>(want, std::max(1, n / abyss::kTile)));
+        }
     }
     if (S > 1) {
         const double per = (double)nt * ((double)cap * 4.0 + 6 * 8.0 + 4.0);

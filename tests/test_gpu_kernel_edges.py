@@ -46,3 +46,30 @@ def test_derivs23_edges(n, m, ref):
     err = np.abs(got - want).reshape(-1, 2, 6) / scale
     say(f"  max err = {err.max():.3e}")
     assert np.isfinite(got).all() and err.max() <= 1e-10
+
+
+@pytest.mark.parametrize("prec", [regf.PREC_SPLIT, regf.PREC_CHECKED, regf.PREC_REFINED])
+@pytest.mark.parametrize("n,m", [(1025, 300), (2049, 2049), (10007, 777), (16385, 4096),
+                                 (65536, 64)])
+def test_short_spans_equal_long_ones(n, m, prec):
+    """A launch of few workgroups takes more, shorter j-splits; with at least
+    four tiles per split the same launch gives the same lists, and sums that
+    differ by the order of their FP64 partials."""
+    say(f"case: spans n={n} m={m} precision={prec}")
+    js = workloads.plummer_kroupa(n, seed=2, k_nb=40)
+    t = np.random.default_rng(m).permutation(n)[:m].astype(np.int32)
+    with regf.Context(device=0, cap=64, precision=prec) as c:
+        c.upload(js.m, js.x, js.v, js.r2)
+        got = [a.copy() for a in c.query(t)]
+        p = c.plan()
+        c.set_tuning(0, max(1, n // 1024), 0, p["lanes_per_target"])
+        want = c.query(t)
+        say(f"  plan {p}, long spans: {c.plan()['j_splits']} splits")
+    assert np.array_equal(got[2], want[2]) and np.array_equal(got[3], want[3])
+    for a, b in zip(got[:2], want[:2]):
+        # the sums have the same FP32 runs and at most 128 + 64 FP64 partials
+        # (200 * 2^-53 of the largest partial, whose ratio to the sum is below
+        # 1e4); a target whose flag changes moves by the checked tolerance
+        rel = np.linalg.norm(a - b, axis=1) / np.linalg.norm(b, axis=1)
+        bad = rel > 1e-9
+        assert rel.max() <= 1e-6 and bad.sum() <= (1 if prec == regf.PREC_CHECKED else 0)
