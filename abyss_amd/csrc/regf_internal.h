@@ -49,6 +49,14 @@ struct CheckFlag {
     const int *tgt = nullptr;
 };
 
+// The caller's unchecked target list of the no-allocation query (tgt null:
+// targets were checked on the host): a finalize gives a target outside
+// [0, n) NaN forces and INT_MIN as its count, and does not flag it.
+struct TargetGuard {
+    const int *tgt = nullptr;
+    int n = 0;
+};
+
 struct Plan {
     int ipl = 1;     // targets per lane
     int splits = 1;  // j-splits (grid.y)
@@ -200,7 +208,8 @@ constexpr int kPrecRecheck = 100;
 hipError_t launch_finalize(const QueryOut &part, int S, int nt, int cap,
                            double *acc, double *adot, int *nnb, int *list,
                            const FinalMirror &mirror, float *spread, hipStream_t st,
-                           const CheckFlag &flag = CheckFlag{});
+                           const CheckFlag &flag = CheckFlag{},
+                           const TargetGuard &guard = TargetGuard{});
 
 // Checked precision.  counters[0] must be 0.  Appends to (fq, fi) the
 // position and j-index of every target q whose a or jdot may be off by
@@ -214,16 +223,6 @@ hipError_t launch_check_flag(const double *acc, const double *adot, const float 
 // split order) and writes them over acc/adot at fq[k].
 hipError_t launch_recheck_finalize(const QueryOut &part, int S, int m, const int *fq,
                                    double *acc, double *adot, hipStream_t st);
-// The same two steps with the flagged count read on the device (*count, as
-// left by launch_check_flag) and no host wait: plan p is for all nt targets
-// (partials [S][nt]); workgroups and waves past the count exit at once.
-// Writes the count to *m_report (host memory) and the results also to the
-// mirror when it is set.
-hipError_t launch_recheck_dev(const JState &js, const int *fi, const int *count, int nt,
-                              const Plan &p, const QueryOut &out, const int *fq, double *acc,
-                              double *adot, const FinalMirror &mirror, int *m_report,
-                              hipStream_t st);
-
 // The recomputation of the first *count targets of fi (count on the device,
 // at most nt): `grid` workgroups loop over the (target block, split) items of
 // plan p (lanes per target, splits and span; 256-record tiles, 4 waves), then

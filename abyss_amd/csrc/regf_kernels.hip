@@ -31,6 +31,8 @@
 #include "../../include/abyss_regf.h"
 #include "regf_internal.h"
 
+#include <limits.h>
+
 namespace abyss {
 namespace {
 
@@ -784,6 +786,17 @@ __device__ __forceinline__ bool check_rule(float sa, float sj, double ax, double
            (double)sj * k2 > fma(jz, jz, fma(jy, jy, jx * jx));
 }
 
+__device__ __forceinline__ bool bad_target(const TargetGuard &g, int q)
+{
+    return g.tgt && (unsigned)g.tgt[q] >= (unsigned)g.n;
+}
+
+__device__ __forceinline__ void mark_bad(double (&a)[6])
+{
+#pragma unroll
+    for (int c = 0; c < 6; ++c) a[c] = __builtin_nan("");
+}
+
 __device__ __forceinline__ void finalize_body(const QueryOut &part, int S, int nt_stride, int cap,
                                               int q_rel, int q, bool active, int *off,
                                               double *__restrict__ acc,
@@ -791,9 +804,11 @@ __device__ __forceinline__ void finalize_body(const QueryOut &part, int S, int n
                                               int *__restrict__ nnb, int *__restrict__ list,
                                               const FinalMirror &mir = FinalMirror{},
                                               float *__restrict__ spread = nullptr,
-                                              const CheckFlag &flag = CheckFlag{})
+                                              const CheckFlag &flag = CheckFlag{},
+                                              const TargetGuard &guard = TargetGuard{})
 {
     const int lane = threadIdx.x & 63;
+    const bool bad = active && bad_target(guard, q);
 
     double a[6];
     sum_splits(part, S, nt_stride, q_rel, active, a);
@@ -815,13 +830,15 @@ __device__ __forceinline__ void finalize_body(const QueryOut &part, int S, int n
             spread[2 * (size_t)q + 1] = ej;
             // checked precision: flag the target here instead of in a
             // separate pass (the rule of check_flag_kernel)
-            if (flag.counter && check_rule(ea, ej, a[0], a[1], a[2], a[3], a[4], a[5], flag.k2)) {
+            if (flag.counter && !bad &&
+                check_rule(ea, ej, a[0], a[1], a[2], a[3], a[4], a[5], flag.k2)) {
                 const int k = atomicAdd(flag.counter, 1);
                 flag.fq[k] = q;
                 flag.fi[k] = flag.tgt[q];
             }
         }
     }
+    if (bad) mark_bad(a);
 
     int running = 0;
     for (int base = 0; base < S; base += 64) {
@@ -863,8 +880,9 @@ __device__ __forceinline__ void finalize_body(const QueryOut &part, int S, int n
         if (mirror) mir.list[(size_t)q * cap + e] = j;
     }
     if (lane == 0) {
-        nnb[q] = total <= cap ? total : -total;
-        if (mirror) mir.nnb[q] = total <= cap ? total : -total;
+        const int c = bad ? INT_MIN : (total <= cap ? total : -total);
+        nnb[q] = c;
+        if (mirror) mir.nnb[q] = c;
     }
 }
 
@@ -873,13 +891,14 @@ __global__ __launch_bounds__(256) void finalize_kernel(QueryOut part, int S, int
                                                        double *__restrict__ adot,
                                                        int *__restrict__ nnb,
                                                        int *__restrict__ list, FinalMirror mir,
-                                                       float *__restrict__ spread, CheckFlag flag)
+                                                       float *__restrict__ spread, CheckFlag flag,
+                                                       TargetGuard guard)
 {
     extern __shared__ int s_off_all[];   // [4 waves][S + 1]
     const int w = threadIdx.x >> 6;
     const int q = blockIdx.x * 4 + w;
     finalize_body(part, S, nt, cap, q, q, q < nt, s_off_all + w * (S + 1), acc, adot, nnb, list,
-                  mir, spread, flag);
+                  mir, spread, flag, guard);
 }
 
 // finalize_kernel for S <= G j-splits: G lanes per target, 64 / G targets
@@ -895,7 +914,7 @@ __global__ __launch_bounds__(256) void finalize_group_kernel(QueryOut part, int 
                                                              int *__restrict__ list,
                                                              FinalMirror mir,
                                                              float *__restrict__ spread,
-                                                             CheckFlag flag)
+                                                             CheckFlag flag, TargetGuard guard)
 {
     static_assert(G >= 8 && G <= 64 && (G & (G - 1)) == 0, "a group holds the 6 sums");
     __shared__ int s_off[256 / G][G + 1];
@@ -904,6 +923,7 @@ __global__ __launch_bounds__(256) void finalize_group_kernel(QueryOut part, int 
     const int q = blockIdx.x * (256 / G) + slot;
     const bool active = q < nt;
     const bool mine = active && sub < S;
+    const bool bad = active && bad_target(guard, q);
     const size_t o = (size_t)sub * nt + q;
     double a[6];
 #pragma unroll
@@ -934,13 +954,15 @@ __global__ __launch_bounds__(256) void finalize_group_kernel(QueryOut part, int 
         if (active && sub == 0) {
             spread[2 * (size_t)q + 0] = ea;
             spread[2 * (size_t)q + 1] = ej;
-            if (flag.counter && check_rule(ea, ej, a[0], a[1], a[2], a[3], a[4], a[5], flag.k2)) {
+            if (flag.counter && !bad &&
+                check_rule(ea, ej, a[0], a[1], a[2], a[3], a[4], a[5], flag.k2)) {
                 const int k = atomicAdd(flag.counter, 1);
                 flag.fq[k] = q;
                 flag.fi[k] = flag.tgt[q];
             }
         }
     }
+    if (bad) mark_bad(a);
 
     // split offsets of this target's list entries: a prefix over its group
     const int c0 = mine ? part.cnt[o] : 0;
@@ -979,8 +1001,9 @@ __global__ __launch_bounds__(256) void finalize_group_kernel(QueryOut part, int 
         if (mirror) mir.list[(size_t)q * cap + e] = j;
     }
     if (sub == 0) {
-        nnb[q] = total <= cap ? total : -total;
-        if (mirror) mir.nnb[q] = total <= cap ? total : -total;
+        const int c = bad ? INT_MIN : (total <= cap ? total : -total);
+        nnb[q] = c;
+        if (mirror) mir.nnb[q] = c;
     }
 }
 
@@ -1015,25 +1038,6 @@ __global__ __launch_bounds__(256) void check_flag_kernel(const double *__restric
         fq[k] = q;
         fi[k] = tgt[q];
     }
-}
-
-// The recomputation with the flagged count read on the device (the
-// no-allocation query: no host wait).  The grid covers every target; a
-// workgroup whose
-// target block starts at or past the count exits before its first barrier.
-// Partials are indexed s * nt_stride + k.
-template <int JL>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5, 8)))
-void recheck_kernel_dev(JState js, const int *__restrict__ tgt, const int *__restrict__ count,
-                        int nt_stride, int jspan, QueryOut out, int gx, int splits)
-{
-    __shared__ double2 s_pos[2][kTile * 3];
-    __shared__ double s_m[2][kTile];
-    const int m = *count;
-    int bx, s;
-    xcd_place(blockIdx.x, gx * splits, gx, bx, s);
-    if (bx * (4 * (64 / JL)) >= m) return;   // the whole workgroup
-    regf_body_jl<JL, 3>(js, tgt, m, jspan, out, 0, 0, bx, s, 0, nt_stride, s_pos, s_m);
 }
 
 // The recomputation with the flagged count read on the device, as a
@@ -1429,24 +1433,25 @@ hipError_t launch_regf(const JState &js, const int *tgt, int nt, const Plan &p,
 
 hipError_t launch_finalize(const QueryOut &part, int S, int nt, int cap, double *acc,
                            double *adot, int *nnb, int *list, const FinalMirror &mirror,
-                           float *spread, hipStream_t st, const CheckFlag &flag)
+                           float *spread, hipStream_t st, const CheckFlag &flag,
+                           const TargetGuard &guard)
 {
     if (spread && !part.spread) return hipErrorInvalidValue;
     if (flag.counter && !spread) return hipErrorInvalidValue;
     if (S <= 8) {
         hipLaunchKernelGGL(finalize_group_kernel<8>, dim3((nt + 31) / 32), dim3(256), 0, st, part,
-                           S, nt, cap, acc, adot, nnb, list, mirror, spread, flag);
+                           S, nt, cap, acc, adot, nnb, list, mirror, spread, flag, guard);
         return hipGetLastError();
     }
     if (S <= 16) {
         hipLaunchKernelGGL(finalize_group_kernel<16>, dim3((nt + 15) / 16), dim3(256), 0, st, part,
-                           S, nt, cap, acc, adot, nnb, list, mirror, spread, flag);
+                           S, nt, cap, acc, adot, nnb, list, mirror, spread, flag, guard);
         return hipGetLastError();
     }
     dim3 grid((nt + 3) / 4);
     const size_t lds = 4 * (size_t)(S + 1) * sizeof(int);
     hipLaunchKernelGGL(finalize_kernel, grid, dim3(256), lds, st, part, S, nt, cap, acc, adot, nnb,
-                       list, mirror, spread, flag);
+                       list, mirror, spread, flag, guard);
     return hipGetLastError();
 }
 
@@ -1464,31 +1469,6 @@ hipError_t launch_recheck_finalize(const QueryOut &part, int S, int m, const int
 {
     hipLaunchKernelGGL(recheck_finalize_kernel, dim3((m + 3) / 4), dim3(256), 0, st, part, S, m,
                        m, (const int *)nullptr, (int *)nullptr, fq, acc, adot, FinalMirror{});
-    return hipGetLastError();
-}
-
-hipError_t launch_recheck_dev(const JState &js, const int *fi, const int *count, int nt,
-                              const Plan &p, const QueryOut &out, const int *fq, double *acc,
-                              double *adot, const FinalMirror &mirror, int *m_report,
-                              hipStream_t st)
-{
-    if ((p.jl != 4 && p.jl != 16 && p.jl != 64) || p.tile != kTile || p.wpb != 4)
-        return hipErrorInvalidValue;
-    if ((long long)p.grid_x * p.splits > 0x7fffffffLL) return hipErrorInvalidValue;
-    dim3 grid(p.grid_x * p.splits);
-    if (p.jl == 4)
-        hipLaunchKernelGGL(recheck_kernel_dev<4>, grid, dim3(kBlock), 0, st, js, fi, count, nt,
-                           p.jspan, out, p.grid_x, p.splits);
-    else if (p.jl == 16)
-        hipLaunchKernelGGL(recheck_kernel_dev<16>, grid, dim3(kBlock), 0, st, js, fi, count, nt,
-                           p.jspan, out, p.grid_x, p.splits);
-    else
-        hipLaunchKernelGGL(recheck_kernel_dev<64>, grid, dim3(kBlock), 0, st, js, fi, count, nt,
-                           p.jspan, out, p.grid_x, p.splits);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(recheck_finalize_kernel, dim3((nt + 3) / 4), dim3(256), 0, st, out,
-                       p.splits, nt, 0, count, m_report, fq, acc, adot, mirror);
     return hipGetLastError();
 }
 

@@ -462,6 +462,23 @@ double check_k2(abyss_ctx_t c)
     return ratio * ratio;
 }
 
+// Plan and grid of the recomputation that loops over a count read on the
+// device, for nt targets of which a typical 1/16 is flagged, with at most
+// max_splits j-splits.
+Plan plan_recheck_loop(abyss_ctx_t c, int nt, int n, int max_splits, int *grid)
+{
+    Plan rp = plan_for(c, std::max(1, nt / 16), n, ABYSS_PREC_REFINED, 0, false);
+    const int tiles = (n + abyss::kTile - 1) / abyss::kTile;
+    rp.splits = std::min(tiles, max_splits);
+    rp.jspan = (tiles + rp.splits - 1) / rp.splits * abyss::kTile;
+    rp.splits = (n + rp.jspan - 1) / rp.jspan;
+    const int tpb = 4 * (64 / rp.jl);
+    const int cu = c->cu_count > 0 ? c->cu_count : 256;
+    const long long items = (long long)((nt + tpb - 1) / tpb) * rp.splits;
+    *grid = (int)std::min<long long>(items, 5LL * cu);
+    return rp;
+}
+
 // After a checked launch's force and finalize: flags the targets whose a or
 // jdot may miss the tolerance (unless the finalize of a split launch has
 // flagged them: `flagged`) and recomputes them with FP64 terms over the
@@ -484,15 +501,8 @@ int recheck(abyss_ctx_t c, bool flagged)
         // the actual one.  Its items are short (j-ranges of 1 tile where N
         // allows, up to 256 splits), since a few flagged targets give few
         // items and each item's tiles run one after another.
-        Plan rp = plan_for(c, std::max(1, c->nt / 16), c->n, ABYSS_PREC_REFINED, 0, false);
-        const int tiles = (c->n + abyss::kTile - 1) / abyss::kTile;
-        rp.splits = std::min(tiles, kRecheckLoopSplits);
-        rp.jspan = (tiles + rp.splits - 1) / rp.splits * abyss::kTile;
-        rp.splits = (c->n + rp.jspan - 1) / rp.jspan;
-        const int tpb = 4 * (64 / rp.jl);
-        const int cu = c->cu_count > 0 ? c->cu_count : 256;
-        const long long items = (long long)((c->nt + tpb - 1) / tpb) * rp.splits;
-        const int grid = (int)std::min<long long>(items, 5LL * cu);
+        int grid = 0;
+        const Plan rp = plan_recheck_loop(c, c->nt, c->n, kRecheckLoopSplits, &grid);
         QueryOut rpart;
         int rc = ensure_recheck_scratch(c, (size_t)rp.splits * c->nt, &rpart);
         if (rc != ABYSS_OK) return rc;
@@ -1154,27 +1164,27 @@ int noalloc_init(int device, char **ptr, int *cu)
 }
 
 // FP32 masses (the rounding of the context's upload) and the checked target
-// copy: an index outside [0, n) becomes 0 in the copy and is counted.
+// copy: an index outside [0, n) becomes 0 in the copy.  Zeroes the flagged
+// count (nothing reads it before the force kernel).
 __global__ void noalloc_prep_kernel(const double *__restrict__ m, float *__restrict__ m32, int n,
                                     const int *__restrict__ tgt, int *__restrict__ tgt_s, int nt,
-                                    int *__restrict__ bad)
+                                    int *__restrict__ count)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0) *count = 0;
     if (i < n) m32[i] = (float)m[i];
     if (i < nt) {
         const int t = tgt[i];
-        const bool ok = t >= 0 && t < n;
-        tgt_s[i] = ok ? t : 0;
-        if (!ok) atomicAdd(bad, 1);
+        tgt_s[i] = t >= 0 && t < n ? t : 0;
     }
 }
 
-// Results of targets outside [0, n): NaN forces and INT_MIN as the count.
+// One-split launches: results of targets outside [0, n), NaN forces and
+// INT_MIN as the count (a split launch's finalize writes them itself).
 __global__ void noalloc_mark_kernel(const int *__restrict__ tgt, int nt, int n,
-                                    const int *__restrict__ bad, double *__restrict__ acc,
-                                    double *__restrict__ adot, int *__restrict__ nnb)
+                                    double *__restrict__ acc, double *__restrict__ adot,
+                                    int *__restrict__ nnb)
 {
-    if (*bad == 0) return;
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= nt) return;
     const int t = tgt[q];
@@ -1243,7 +1253,7 @@ int abyss_query_noalloc(int device, int n, const double *jset, int nt, const int
     const size_t S = (size_t)p.splits, t = (size_t)nt;
 
     Carve cv{base};
-    int *counters = reinterpret_cast<int *>(cv.take(256));   // [0] flagged, [1] bad targets
+    int *counters = reinterpret_cast<int *>(cv.take(256));   // [0] flagged
     int *tgt_s = reinterpret_cast<int *>(cv.take(t * sizeof(int)));
     float *m32 = reinterpret_cast<float *>(cv.take((size_t)n * sizeof(float)));
     QueryOut part{};
@@ -1262,16 +1272,18 @@ int abyss_query_noalloc(int device, int n, const double *jset, int nt, const int
         fi = reinterpret_cast<int *>(cv.take(t * sizeof(int)));
     }
     if (cv.used > ABYSS_NOALLOC_SCRATCH_BYTES) return done(ABYSS_ERR_SCRATCH_LIMIT);
-    // the recomputation of checked precision: planned for every target (the
-    // flagged count stays on the device), its splits bounded by what is left
+    // the recomputation of checked precision loops over the flagged count,
+    // which stays on the device; its splits are bounded by what is left
     Plan rp{};
     QueryOut rpart{};
+    int rgrid = 0;
     if (checked) {
         const size_t row = 2 * 3 * sizeof(double) + sizeof(int);
         const size_t left = ABYSS_NOALLOC_SCRATCH_BYTES - cv.used;
         if (left < t * row + 3 * 256) return done(ABYSS_ERR_SCRATCH_LIMIT);
-        tmp.scratch_limit = left - 3 * 256;
-        rp = plan_for(&tmp, nt, n, ABYSS_PREC_REFINED, 0, false);
+        const size_t fit = (left - 3 * 256) / (t * row);
+        rp = plan_recheck_loop(&tmp, nt, n, (int)std::min<size_t>(fit, kRecheckLoopSplits),
+                               &rgrid);
         const size_t rows = (size_t)rp.splits * t;
         rpart.acc = reinterpret_cast<double *>(cv.take(rows * 3 * sizeof(double)));
         rpart.adot = reinterpret_cast<double *>(cv.take(rows * 3 * sizeof(double)));
@@ -1295,30 +1307,36 @@ int abyss_query_noalloc(int device, int n, const double *jset, int nt, const int
     do {                                             \
         if ((call) != hipSuccess) return done(ABYSS_ERR_HIP); \
     } while (0)
-    NACHK(abyss::launch_batch_reset(counters, st));   // both counters := 0
+    // Small queries are bound by the chain of dependent kernels: five (three
+    // in split precision) with the count's reset in the first, and the
+    // flagging and the marking of bad targets in the merge; eight took
+    // 51.2 us at N = 10007 with 777 targets, five take 41.1 us.
     const int w = std::max(n, nt);
     hipLaunchKernelGGL(noalloc_prep_kernel, dim3((w + 255) / 256), dim3(256), 0, st, js.m, m32, n,
-                       targets, tgt_s, nt, counters + 1);
+                       targets, tgt_s, nt, counters);
     NACHK(hipGetLastError());
     QueryOut fin{acc, adot, nnb, list};
     fin.spread = spread;
-    if (S == 1) {
-        NACHK(abyss::launch_regf(js, tgt_s, nt, p, fin, cap, kprec, st));
-    } else {
-        NACHK(abyss::launch_regf(js, tgt_s, nt, p, part, cap, kprec, st));
+    const double ratio = ABYSS_CHECK_ERR_SCALE / 1.0e-6;
+    const double k2 = ratio * ratio;
+    NACHK(abyss::launch_regf(js, tgt_s, nt, p, S == 1 ? fin : part, cap, kprec, st));
+    if (S > 1) {
+        abyss::CheckFlag flag;
+        if (checked) flag = abyss::CheckFlag{k2, counters, fq, fi, tgt_s};
         NACHK(abyss::launch_finalize(part, p.splits, nt, cap, acc, adot, nnb, list,
-                                     abyss::FinalMirror{}, spread, st));
+                                     abyss::FinalMirror{}, spread, st, flag,
+                                     abyss::TargetGuard{targets, n}));
+    } else if (checked) {
+        NACHK(abyss::launch_check_flag(acc, adot, spread, tgt_s, nt, k2, counters, fq, fi, st));
     }
-    if (checked) {
-        const double ratio = ABYSS_CHECK_ERR_SCALE / 1.0e-6;
-        NACHK(abyss::launch_check_flag(acc, adot, spread, tgt_s, nt, ratio * ratio, counters, fq,
-                                       fi, st));
-        NACHK(abyss::launch_recheck_dev(js, fi, counters, nt, rp, rpart, fq, acc, adot,
-                                        abyss::FinalMirror{}, nullptr, st));
+    if (checked)
+        NACHK(abyss::launch_recheck_loop(js, fi, counters, nt, rp, rgrid, rpart, fq, acc, adot,
+                                         nullptr, st));
+    if (S == 1) {
+        hipLaunchKernelGGL(noalloc_mark_kernel, dim3((nt + 255) / 256), dim3(256), 0, st, targets,
+                           nt, n, acc, adot, nnb);
+        NACHK(hipGetLastError());
     }
-    hipLaunchKernelGGL(noalloc_mark_kernel, dim3((nt + 255) / 256), dim3(256), 0, st, targets,
-                       nt, n, counters + 1, acc, adot, nnb);
-    NACHK(hipGetLastError());
 #undef NACHK
     return done(ABYSS_OK);
 }

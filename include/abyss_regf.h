@@ -504,8 +504,8 @@ unsigned long long abyss_srv_cluster_footprint(abyss_srv_t srv, int n);
  * abyss_ctx_set_targets + abyss_ctx_launch on a context holding the same
  * j-set, with the same precision and scratch limit ABYSS_NOALLOC_SPLIT_BYTES
  * (checked precision: targets it recomputes agree to FP64 rounding, since
- * the recomputation here is planned for every target and reads the flagged
- * count on the device).
+ * the recomputation here reads the flagged count on the device and splits
+ * j by what the scratch holds).
  *   jset: device SoA of n particles, 8 arrays of n doubles
  *         [x | y | z | vx | vy | vz | m | r_nb^2];
  *   targets: device int[nt], indices into the j-set (0 < nt <= n);

@@ -73,3 +73,27 @@ def test_short_spans_equal_long_ones(n, m, prec):
         rel = np.linalg.norm(a - b, axis=1) / np.linalg.norm(b, axis=1)
         bad = rel > 1e-9
         assert rel.max() <= 1e-6 and bad.sum() <= (1 if prec == regf.PREC_CHECKED else 0)
+
+
+@pytest.mark.parametrize("prec", [regf.PREC_SPLIT, regf.PREC_CHECKED])
+@pytest.mark.parametrize("n,m", [(1024, 300), (4096, 600), (16385, 601), (65536, 300)])
+def test_noalloc_bad_targets_in_every_merge(n, m, prec):
+    """One split, and the merges of up to 8, up to 16 and more splits: bad
+    targets get NaN and INT_MIN and are not recomputed, the others are as on
+    a list that holds target 0 in their place."""
+    from .test_zz_no_alloc import Hip, assert_same, context_query, device_jset, noalloc_query
+    js = workloads.plummer_kroupa(n, seed=2, k_nb=40)
+    t = np.random.default_rng(m).permutation(n)[:m].astype(np.int32)
+    bad = np.array([0, 5, 17, m - 1])
+    t[bad] = [n, -1, np.iinfo(np.int32).min, np.iinfo(np.int32).max]
+    hip = Hip()
+    try:
+        got = noalloc_query(hip, device_jset(hip, js), n, t, 64, prec)
+    finally:
+        hip.free()
+    t0 = t.copy()
+    t0[bad] = 0
+    assert np.isnan(got[0][bad]).all() and np.isnan(got[1][bad]).all()
+    assert (got[2][bad] == np.iinfo(np.int32).min).all()
+    good = np.setdiff1d(np.arange(m), bad)
+    assert_same(got, context_query(js, t0, 64, prec), 64, prec, rows=good)
