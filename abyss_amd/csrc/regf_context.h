@@ -38,18 +38,24 @@ struct abyss_ctx_s {
     // rows [nt][cap]; the pointers below are views of d_out / h_out for the
     // current nt (the host mirror holds rows only up to the one-copy size)
     char *d_out = nullptr, *h_out = nullptr;
+    size_t h_row_bytes = 0;   // list rows h_out has room for
     double *d_acc = nullptr, *d_adot = nullptr;
     int *d_nnb = nullptr, *d_list = nullptr;
     double *h_res = nullptr;  // acc then adot
     int *h_nnb = nullptr, *h_rows = nullptr;
-    // h_out is mapped, coherent pinned memory; for small split launches the
-    // finalize also writes the results there (device view `mirror`), and
-    // mirror_valid tells fetch that no copy is needed
+    // h_out is mapped, coherent pinned memory; the last kernels of small
+    // launches also write the results there (device view `mirror`; for one
+    // split it is where the views above point), and mirror_valid tells fetch
+    // that no copy is needed
     char *h_out_dev = nullptr;
     abyss::FinalMirror mirror{};
     bool mirror_valid = false;
-    int *h_list = nullptr;    // pinned, populated columns of larger results
+    int *h_list = nullptr;    // mapped pinned rows of larger results
+    int *h_list_dev = nullptr;   // their device address
     size_t h_list_bytes = 0;
+    // one event per chunk of a large fetch
+    static constexpr int kFetchChunks = 16;
+    hipEvent_t fev[kFetchChunks] = {};
 
     // device-resident particle state (regf_state.hip): SoA x,v,a,adot (3n
     // each), t, m, r2 (n each); staging for incremental updates
@@ -136,7 +142,9 @@ int ctx_fetch_on_stream(abyss_ctx_t c, hipStream_t st, double *acc, double *adot
 // Device bytes a context holds (j-set, targets, outputs, scratch).
 unsigned long long ctx_device_bytes(abyss_ctx_t c);
 // abyss_ctx_launch without keeping the resident lists (force kernels only).
-int ctx_launch_force(abyss_ctx_t c);
+// to_host: a fetch follows, so blocks of up to kQueryMirrorTargets targets
+// also write their results to mapped host memory.
+int ctx_launch_force(abyss_ctx_t c, bool to_host = false);
 // After a launch: copies its neighbour rows into the resident per-particle
 // lists when they are enabled (no-op otherwise).
 int keep_launch_lists(abyss_ctx_t c);

@@ -211,6 +211,11 @@ hipError_t launch_finalize(const QueryOut &part, int S, int nt, int cap,
                            const CheckFlag &flag = CheckFlag{},
                            const TargetGuard &guard = TargetGuard{});
 
+// Copies the populated entries of list rows [q0, q1) (row stride cap) to
+// `rows` (mapped host memory, row stride `width` >= every populated count).
+hipError_t launch_pack_rows(const int *list, const int *nnb, int cap, int q0, int q1, int *rows,
+                            int width, hipStream_t st);
+
 // Checked precision.  counters[0] must be 0.  Appends to (fq, fi) the
 // position and j-index of every target q whose a or jdot may be off by
 // more than the tolerance: spread[q][0] * k2 > |acc[q]|^2 or spread[q][1] *
@@ -220,9 +225,10 @@ hipError_t launch_check_flag(const double *acc, const double *adot, const float 
                              const int *tgt, int nt, double k2, int *counters, int *fq, int *fi,
                              hipStream_t st);
 // Sums the recomputation's S partials of each of the m flagged targets (in
-// split order) and writes them over acc/adot at fq[k].
+// split order) and writes them over acc/adot (and the mirror's) at fq[k].
 hipError_t launch_recheck_finalize(const QueryOut &part, int S, int m, const int *fq,
-                                   double *acc, double *adot, hipStream_t st);
+                                   double *acc, double *adot, const FinalMirror &mirror,
+                                   hipStream_t st);
 // The recomputation of the first *count targets of fi (count on the device,
 // at most nt): `grid` workgroups loop over the (target block, split) items of
 // plan p (lanes per target, splits and span; 256-record tiles, 4 waves), then
@@ -230,6 +236,7 @@ hipError_t launch_recheck_finalize(const QueryOut &part, int S, int m, const int
 // *m_report (mapped host memory) when it is set.
 hipError_t launch_recheck_loop(const JState &js, const int *fi, const int *count, int nt,
                                const Plan &p, int grid, const QueryOut &out, const int *fq,
-                               double *acc, double *adot, int *m_report, hipStream_t st);
+                               double *acc, double *adot, const FinalMirror &mirror,
+                               int *m_report, hipStream_t st);
 
 }  // namespace abyss

@@ -442,7 +442,7 @@ int abyss_ctx_regular_step(abyss_ctx_t c, int nt, const int *targets, const doub
     if (hipMemcpyAsync(c->d_irr, c->h_irr, in_bytes, hipMemcpyHostToDevice, c->stream) !=
         hipSuccess)
         return ABYSS_ERR_HIP;
-    rc = abyss::ctx_launch_force(c);
+    rc = abyss::ctx_launch_force(c, true);   // the fetch below
     if (rc != ABYSS_OK) return rc;
     const double *d_in = reinterpret_cast<const double *>(c->d_irr);
     double *d_out = reinterpret_cast<double *>(c->d_irr) + (size_t)nt * 7;

@@ -1,6 +1,7 @@
 // Host side of a j-set upload: validation of the caller's arrays and the
 // AoS -> SoA pack into the device layout, spread over a small pool of host
-// threads for large N.
+// threads for large N.  The same pool copies large results out of the pinned
+// staging into the caller's arrays.
 //
 // Reference counterpart: the pack loop of _ReceiveFromHost
 // (src/cuda/cuda_my_acceleration.cu:399-405, src_mpi/cuda/
@@ -9,6 +10,7 @@
 #include "regf_pack.h"
 
 #include <math.h>
+#include <string.h>
 
 #include <algorithm>
 #include <atomic>
@@ -231,6 +233,21 @@ PackStatus pack_jset(int n, int j0, int j1, const double *m, const double *x, co
     for (const PackStatus &s : st)   // parts in index order: the first is the lowest
         if (s.index >= 0) return s;
     return {};
+}
+
+int host_parts() { return pool().workers() + 1; }
+
+bool host_run(int parts, const std::function<void(int)> &f) { return pool().run(parts, f); }
+
+void unpack_rows(int k0, int k1, const int *counts, const int *rows, size_t stride, int cap,
+                 int *list)
+{
+    for (int k = k0; k < k1; ++k) {
+        const int c = counts[k];
+        const int n = std::min(c < 0 ? -c : c, cap);
+        if (n > 0)
+            memcpy(list + (size_t)k * cap, rows + (size_t)k * stride, (size_t)n * sizeof(int));
+    }
 }
 
 }  // namespace abyss

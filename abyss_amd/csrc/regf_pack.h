@@ -36,4 +36,16 @@ PackStatus pack_jset_staged(int n, const double *m, const double *x, const doubl
                             const double *r2, double *soa, float *m32,
                             const std::function<void()> &positions_done);
 
+// Host threads a job can run on, the caller's included (1: none started).
+int host_parts();
+// Runs f(0) on the caller and f(1) ... f(parts - 1) on the pool's threads
+// (parts <= host_parts()); returns when all are done.  False, with nothing
+// run, when another caller's job holds the pool.
+bool host_run(int parts, const std::function<void(int)> &f);
+
+// Copies the populated entries (min(|counts[k]|, cap)) of list rows [k0, k1)
+// from `rows` (row stride `stride`) to `list` (row stride cap).
+void unpack_rows(int k0, int k1, const int *counts, const int *rows, size_t stride, int cap,
+                 int *list);
+
 }  // namespace abyss

@@ -21,7 +21,9 @@
 #include <string.h>
 
 #include <algorithm>
+#include <atomic>
 #include <mutex>
+#include <thread>
 
 using abyss::JState;
 using abyss::Plan;
@@ -35,9 +37,25 @@ constexpr size_t kOneTripListBytes = 1u << 20;
 // Up to this many targets the kernels read the target list straight from
 // mapped host memory instead of a device copy (saves one copy per query).
 constexpr int kMappedTargets = 64;
-// a checked block with a mapped mirror runs in FP64 terms in one pass, so no
-// recomputation ever has to update the mirror
-static_assert(abyss::kCheckedDirectMax >= kMappedTargets, "mirrored blocks are direct");
+// A query (launch and fetch in one call) of up to this many targets, with
+// full-width list rows up to this many bytes, has its last kernels write the
+// results into mapped host memory as well, so its fetch is one wait instead
+// of a wait for the counts and a copy of the rows.  Calls before -> after, N
+// / targets: 65536 / 1000 158 -> 132 us, 16385 / 4096 refined 240 -> 182 us
+// (1024 / 1 in place, without the copy: 28 -> 22.5 us).  Above, the rows take
+// longer on the link than a second wait (and pinning them costs 0.1 ms per
+// MB once).
+constexpr int kQueryMirrorTargets = 4096;
+constexpr size_t kQueryMirrorRowBytes = 4u << 20;
+// Larger results come back in chunks of at least this many bytes of rows, so
+// that the host copies one chunk into the caller's rows while the next is on
+// the link; from this many bytes up the copies run on several host threads
+// (one thread copies 20 to 32 GB/s, eight 60 GB/s, the link brings 50 GB/s).
+// N / targets 65536 / 20011: 1827 -> 1406 us per query, 30011 / 30011 split:
+// 1461 -> 1037 us.
+constexpr size_t kFetchChunkBytes = 2u << 20;
+constexpr size_t kUnpackParallelBytes = 1u << 20;
+constexpr int kUnpackParts = 8;
 // Most j-splits of the recomputation that reads its count on the device
 // (scratch: this many rows per target of the block, 52 bytes each).
 constexpr int kRecheckLoopSplits = 256;
@@ -109,7 +127,8 @@ size_t packed_bytes(size_t nt)
 
 // Views of the output block for the current target count: acc, adot, nnb,
 // then the list rows, so that one copy can move every result of a small
-// query.  The host block mirrors the layout up to kOneTripListBytes of rows.
+// query.  The host block mirrors the layout up to the rows a fetch or a
+// query's last kernels put there.
 void set_output_views(abyss_ctx_t c, int nt)
 {
     const size_t n = (size_t)nt;
@@ -117,6 +136,8 @@ void set_output_views(abyss_ctx_t c, int nt)
     c->d_adot = c->d_acc + 3 * n;
     c->d_nnb = reinterpret_cast<int *>(c->d_adot + 3 * n);
     c->d_list = reinterpret_cast<int *>(c->d_out + packed_bytes(n));
+    c->mirror = abyss::FinalMirror{};
+    if (!c->h_out) return;
     c->h_res = reinterpret_cast<double *>(c->h_out);
     c->h_nnb = reinterpret_cast<int *>(c->h_res + 6 * n);
     c->h_rows = reinterpret_cast<int *>(c->h_out + packed_bytes(n));
@@ -127,35 +148,60 @@ void set_output_views(abyss_ctx_t c, int nt)
     c->mirror.list = reinterpret_cast<int *>(c->h_out_dev + packed_bytes(n));
 }
 
-int ensure_outputs(abyss_ctx_t c, int nt)
+// The mapped host block of t_capacity targets' packed results with room for
+// at least `bytes` of list rows (no launch that writes it may be in flight).
+int ensure_host_rows(abyss_ctx_t c, size_t bytes)
 {
-    if ((size_t)nt <= c->t_capacity) {
-        set_output_views(c, nt);
-        return ABYSS_OK;
-    }
-    size_t cap_t = grow((size_t)nt);
-    dfree(c->d_tgt); dfree(c->d_out);
-    hfree(c->h_tgt); hfree(c->h_out);
-    c->t_capacity = 0;
-    c->d_list = nullptr;
-    c->h_tgt_dev = c->tgt = nullptr;
+    if (c->h_out && bytes <= c->h_row_bytes) return ABYSS_OK;
+    hfree(c->h_out);
     c->h_out_dev = nullptr;
+    c->h_row_bytes = 0;
     c->mirror = abyss::FinalMirror{};
     c->mirror_valid = false;
-    const size_t rows = cap_t * (size_t)c->cap * sizeof(int);
-    HIPCHK(c, hipMalloc(&c->d_tgt, cap_t * sizeof(int)));
-    HIPCHK(c, hipMalloc(&c->d_out, packed_bytes(cap_t) + rows));
-    HIPCHK(c, hipHostMalloc(&c->h_tgt, cap_t * sizeof(int),
-                            hipHostMallocMapped | hipHostMallocCoherent));
-    void *dev = nullptr;
-    HIPCHK(c, hipHostGetDevicePointer(&dev, c->h_tgt, 0));
-    c->h_tgt_dev = static_cast<const int *>(dev);
-    HIPCHK(c, hipHostMalloc(&c->h_out, packed_bytes(cap_t) + std::min(rows, kOneTripListBytes),
+    // two sizes, so that growing blocks do not pin it again and again
+    const size_t all = c->t_capacity * (size_t)c->cap * sizeof(int);
+    const size_t room =
+        std::max(bytes, std::min(all, bytes > kOneTripListBytes ? kQueryMirrorRowBytes
+                                                                : kOneTripListBytes));
+    HIPCHK(c, hipHostMalloc(&c->h_out, packed_bytes(c->t_capacity) + room,
                             hipHostMallocMapped | hipHostMallocCoherent));
     void *out_dev = nullptr;
     HIPCHK(c, hipHostGetDevicePointer(&out_dev, c->h_out, 0));
     c->h_out_dev = static_cast<char *>(out_dev);
-    c->t_capacity = cap_t;
+    c->h_row_bytes = room;
+    return ABYSS_OK;
+}
+
+int ensure_outputs(abyss_ctx_t c, int nt)
+{
+    if ((size_t)nt > c->t_capacity) {
+        size_t cap_t = grow((size_t)nt);
+        dfree(c->d_tgt); dfree(c->d_out);
+        hfree(c->h_tgt); hfree(c->h_out);
+        c->t_capacity = 0;
+        c->d_list = nullptr;
+        c->h_tgt_dev = c->tgt = nullptr;
+        c->h_out_dev = nullptr;
+        c->h_row_bytes = 0;
+        c->mirror = abyss::FinalMirror{};
+        c->mirror_valid = false;
+        const size_t rows = cap_t * (size_t)c->cap * sizeof(int);
+        HIPCHK(c, hipMalloc(&c->d_tgt, cap_t * sizeof(int)));
+        HIPCHK(c, hipMalloc(&c->d_out, packed_bytes(cap_t) + rows));
+        HIPCHK(c, hipHostMalloc(&c->h_tgt, cap_t * sizeof(int),
+                                hipHostMallocMapped | hipHostMallocCoherent));
+        void *dev = nullptr;
+        HIPCHK(c, hipHostGetDevicePointer(&dev, c->h_tgt, 0));
+        c->h_tgt_dev = static_cast<const int *>(dev);
+        c->t_capacity = cap_t;
+    }
+    // a batch member's results may be fetched while other launches run, so
+    // its host block is allocated here; a context's by the launch or the
+    // fetch that uses it, at the size that takes
+    if (c->batch_member) {
+        int rc = ensure_host_rows(c, 0);
+        if (rc != ABYSS_OK) return rc;
+    }
     set_output_views(c, nt);
     return ABYSS_OK;
 }
@@ -439,7 +485,7 @@ int ensure_recheck_scratch(abyss_ctx_t c, size_t rows, QueryOut *rpart)
 
 // The recomputation of m flagged targets (c->chk_fq / chk_fi hold them),
 // planned for m; the stream need not be idle.
-int recompute_flagged(abyss_ctx_t c, int m)
+int recompute_flagged(abyss_ctx_t c, int m, const abyss::FinalMirror &mirror)
 {
     c->n_rechecked = m;
     if (m <= 0) return ABYSS_OK;
@@ -451,7 +497,7 @@ int recompute_flagged(abyss_ctx_t c, int m)
     HIPCHK(c, abyss::launch_regf(c->js, c->chk_fi, m, rp, rpart, 0, abyss::kPrecRecheck,
                                  c->stream));
     HIPCHK(c, abyss::launch_recheck_finalize(rpart, rp.splits, m, c->chk_fq, c->d_acc, c->d_adot,
-                                             c->stream));
+                                             mirror, c->stream));
     return ABYSS_OK;
 }
 
@@ -484,9 +530,9 @@ Plan plan_recheck_loop(abyss_ctx_t c, int nt, int n, int max_splits, int *grid)
 // flagged them: `flagged`) and recomputes them with FP64 terms over the
 // same regular set: the flagged count is read back (a host wait) and the
 // recomputation planned for it.  (Blocks small enough to skip that wait run
-// in FP64 terms in one pass instead, Plan::fp64_terms; a finalize mirror is
-// written only for them, so the recomputed targets never have to update it.)
-int recheck(abyss_ctx_t c, bool flagged)
+// in FP64 terms in one pass instead, Plan::fp64_terms.)  The recomputed
+// targets' results also go to the mirror when it is set.
+int recheck(abyss_ctx_t c, bool flagged, const abyss::FinalMirror &mirror)
 {
     if (!flagged) {
         // one-split launches: a flag pass over the final results (the force
@@ -507,7 +553,7 @@ int recheck(abyss_ctx_t c, bool flagged)
         int rc = ensure_recheck_scratch(c, (size_t)rp.splits * c->nt, &rpart);
         if (rc != ABYSS_OK) return rc;
         HIPCHK(c, abyss::launch_recheck_loop(c->js, c->chk_fi, c->chk_counters, c->nt, rp, grid,
-                                             rpart, c->chk_fq, c->d_acc, c->d_adot,
+                                             rpart, c->chk_fq, c->d_acc, c->d_adot, mirror,
                                              c->h_chk_dev + 1, c->stream));
         c->recheck_pending = true;
         return ABYSS_OK;
@@ -515,7 +561,7 @@ int recheck(abyss_ctx_t c, bool flagged)
     HIPCHK(c, hipMemcpyAsync(c->h_chk, c->chk_counters, sizeof(int), hipMemcpyDeviceToHost,
                              c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    return recompute_flagged(c, c->h_chk[0]);
+    return recompute_flagged(c, c->h_chk[0], mirror);
 }
 
 // Force-kernel timing: adds up the event pairs recorded so far (waits for
@@ -548,6 +594,11 @@ void release_all(abyss_ctx_t c)
     hfree(c->h_state); hfree(c->h_upd); hfree(c->h_irr);
     hfree(c->h_tgt); hfree(c->h_out); hfree(c->h_list);
     for (hipEvent_t &e : c->kev)
+        if (e) {
+            (void)hipEventDestroy(e);
+            e = nullptr;
+        }
+    for (hipEvent_t &e : c->fev)
         if (e) {
             (void)hipEventDestroy(e);
             e = nullptr;
@@ -905,7 +956,7 @@ namespace abyss {
 
 int ctx_ensure_check(abyss_ctx_t c, int nt, int S) { return ensure_check(c, nt, S); }
 
-int ctx_launch_force(abyss_ctx_t c)
+int ctx_launch_force(abyss_ctx_t c, bool to_host)
 {
     if (!c) return ABYSS_ERR_INVALID_ARG;
     if (c->n <= 0) return set_detail(c, ABYSS_ERR_NO_JSET, "no j-set uploaded");
@@ -929,6 +980,28 @@ int ctx_launch_force(abyss_ctx_t c)
         int rc = ensure_check(c, c->nt, p.splits);
         if (rc != ABYSS_OK) return rc;
     }
+    // Small results also go straight into the mapped host block, so that a
+    // following fetch needs no copy: written by the merge of the splits (and
+    // the recomputation after it), or, for a small one-split launch, by the
+    // force kernel itself, whose results then live there.
+    const size_t row_bytes = (size_t)c->nt * c->cap * sizeof(int);
+    const bool small = c->nt <= kMappedTargets && row_bytes <= kOneTripListBytes;
+    const bool mirrored = !c->batch_member &&
+                          (small || (to_host && p.splits > 1 && c->nt <= kQueryMirrorTargets &&
+                                     row_bytes <= kQueryMirrorRowBytes));
+    if (mirrored) {
+        int rc = ensure_host_rows(c, row_bytes);
+        if (rc != ABYSS_OK) return rc;
+    }
+    set_output_views(c, c->nt);
+    const bool in_place = mirrored && p.splits == 1 && !checked;
+    if (in_place) {
+        c->d_acc = c->mirror.acc;
+        c->d_adot = c->mirror.adot;
+        c->d_nnb = c->mirror.nnb;
+        c->d_list = c->mirror.list;
+    }
+    const abyss::FinalMirror mirror = mirrored && !in_place ? c->mirror : abyss::FinalMirror{};
     QueryOut fin{c->d_acc, c->d_adot, c->d_nnb, c->d_list};
     QueryOut part = c->part;
     if (checked) {
@@ -954,11 +1027,6 @@ int ctx_launch_force(abyss_ctx_t c)
         c->kev_used += 1;
     }
     if (p.splits > 1) {
-        // small results also go straight into the mapped host block, so a
-        // following fetch needs no copy (a checked recomputation updates it
-        // too)
-        const bool mirror = c->nt <= kMappedTargets && !c->batch_member &&
-                            (size_t)c->nt * c->cap * sizeof(int) <= kOneTripListBytes;
         abyss::CheckFlag flag;
         if (checked) {
             flag.k2 = check_k2(c);
@@ -968,13 +1036,12 @@ int ctx_launch_force(abyss_ctx_t c)
             flag.tgt = c->tgt;
         }
         HIPCHK(c, abyss::launch_finalize(part, p.splits, c->nt, c->cap, c->d_acc, c->d_adot,
-                                         c->d_nnb, c->d_list,
-                                         mirror ? c->mirror : abyss::FinalMirror{},
-                                         fin.spread, c->stream, flag));
-        c->mirror_valid = mirror;
+                                         c->d_nnb, c->d_list, mirror, fin.spread, c->stream,
+                                         flag));
     }
+    c->mirror_valid = in_place || (mirrored && p.splits > 1);
     if (checked) {
-        int rc = recheck(c, p.splits > 1);
+        int rc = recheck(c, p.splits > 1, mirror);
         if (rc != ABYSS_OK) return rc;
         c->spread_valid = true;
     }
@@ -987,16 +1054,22 @@ int ctx_launch_force(abyss_ctx_t c)
 
 }  // namespace abyss
 
-extern "C" {
+namespace {
 
-int abyss_ctx_launch(abyss_ctx_t c)
+int launch_and_keep(abyss_ctx_t c, bool to_host)
 {
-    int rc = abyss::ctx_launch_force(c);
+    int rc = abyss::ctx_launch_force(c, to_host);
     if (rc != ABYSS_OK) return rc;
     rc = abyss::keep_launch_lists(c);
     if (rc != ABYSS_OK) return set_detail(c, rc, "keeping resident neighbour lists failed");
     return ABYSS_OK;
 }
+
+}  // namespace
+
+extern "C" {
+
+int abyss_ctx_launch(abyss_ctx_t c) { return launch_and_keep(c, false); }
 
 int abyss_ctx_sync(abyss_ctx_t c)
 {
@@ -1035,6 +1108,60 @@ int abyss_ctx_kernel_timing(abyss_ctx_t c, double *force_ms, long long *launches
 
 namespace abyss {
 
+namespace {
+
+// Copies the host block's acc, adot and counts and the list rows into the
+// caller's arrays; with chunks > 0 the rows of chunk k are there once
+// c->fev[k] has completed.  Large results are copied by several host
+// threads, each a slice of every chunk: one waits for the events and lets
+// the others (and itself) at the chunks that have arrived.
+hipError_t unpack_results(abyss_ctx_t c, int chunks, const int *rows, size_t stride,
+                          size_t list_bytes, double *acc, double *adot, int *nnb, int *list)
+{
+    const int nt = c->nt, cap = c->cap;
+    const int nchunk = std::max(chunks, 1);
+    std::atomic<int> ready{chunks > 0 ? 0 : nchunk};
+    hipError_t err = hipSuccess;   // written by part 0 before it opens the last chunk
+    int parts = 1;
+    const auto part = [&](int p) {
+        const auto slice = [&](int a, int b, int *lo, int *hi) {
+            *lo = a + (int)((long long)(b - a) * p / parts);
+            *hi = a + (int)((long long)(b - a) * (p + 1) / parts);
+        };
+        int lo = 0, hi = 0;
+        slice(0, nt, &lo, &hi);
+        const size_t n3 = 3 * (size_t)(hi - lo), o3 = 3 * (size_t)lo;
+        memcpy(acc + o3, c->h_res + o3, n3 * sizeof(double));
+        memcpy(adot + o3, c->h_res + 3 * (size_t)nt + o3, n3 * sizeof(double));
+        memcpy(nnb + lo, c->h_nnb + lo, (size_t)(hi - lo) * sizeof(int));
+        for (int k = 0; k < nchunk; ++k) {
+            if (p == 0 && chunks > 0) {
+                const hipError_t e = err == hipSuccess ? hipEventSynchronize(c->fev[k]) : err;
+                if (e != hipSuccess) err = e;
+                ready.store(e == hipSuccess ? k + 1 : -1, std::memory_order_release);
+            }
+            int r = ready.load(std::memory_order_acquire);
+            while (r >= 0 && r <= k) {
+                std::this_thread::yield();
+                r = ready.load(std::memory_order_acquire);
+            }
+            if (r < 0) return;   // a failed wait: nothing more arrives
+            slice((int)((long long)nt * k / nchunk), (int)((long long)nt * (k + 1) / nchunk), &lo,
+                  &hi);
+            abyss::unpack_rows(lo, hi, c->h_nnb, rows, stride, cap, list);
+        }
+    };
+    if (list_bytes >= kUnpackParallelBytes) {
+        parts = std::min(abyss::host_parts(), kUnpackParts);
+        if (parts > 1 && abyss::host_run(parts, part)) return err;
+        parts = 1;
+    }
+    part(0);
+    return err;
+}
+
+}  // namespace
+
 int ctx_fetch_on_stream(abyss_ctx_t c, hipStream_t st, double *acc, double *adot, int *nnb,
                         int *list)
 {
@@ -1045,55 +1172,78 @@ int ctx_fetch_on_stream(abyss_ctx_t c, hipStream_t st, double *acc, double *adot
     HIPCHK(c, hipSetDevice(c->device));
     const int nt = c->nt;
     const int cap = c->cap;
-    // Small results: acc, adot, counts and the full list rows are one
-    // contiguous block, moved by one copy.  Larger ones: the counts first,
-    // then only the populated list columns.
+    // Mirrored results are in the host block already.  Other small ones:
+    // acc, adot, counts and the full list rows are one contiguous block,
+    // moved by one copy.  Larger ones: the counts first, then only the
+    // populated list entries, in chunks.
     const size_t full_bytes = (size_t)nt * cap * sizeof(int);
-    const bool one_trip = full_bytes <= kOneTripListBytes;
-    if (c->mirror_valid && st == c->stream) {
-        // the launch's finalize already wrote every result into h_out
-        HIPCHK(c, hipStreamSynchronize(st));
-    } else {
+    const bool mirrored = c->mirror_valid && st == c->stream;
+    const bool one_trip = mirrored || full_bytes <= kOneTripListBytes;
+    if (!mirrored) {
+        int rc = ensure_host_rows(c, one_trip ? full_bytes : 0);
+        if (rc != ABYSS_OK) return rc;
+        set_output_views(c, nt);
+    }
+    if (!mirrored)
         HIPCHK(c, hipMemcpyAsync(c->h_out, c->d_out,
                                  one_trip ? packed_bytes((size_t)nt) + full_bytes
                                           : (size_t)nt * (6 * sizeof(double) + sizeof(int)),
                                  hipMemcpyDeviceToHost, st));
-        HIPCHK(c, hipStreamSynchronize(st));
-    }
+    HIPCHK(c, hipStreamSynchronize(st));
     // populated width and overflow count, from the counts on the host
     int width = 0, overflowed = 0;
+    size_t entries = 0;
     for (int k = 0; k < nt; ++k) {
         const int cnt = c->h_nnb[k];
+        const int n = std::min(cnt < 0 ? -cnt : cnt, cap);
         overflowed += cnt < 0;
-        width = std::max(width, std::min(cnt < 0 ? -cnt : cnt, cap));
+        width = std::max(width, n);
+        entries += n;
     }
+    const size_t list_bytes = entries * sizeof(int);
     const int *rows = c->h_rows;
-    int stride = cap;   // row stride of `rows`
+    size_t stride = cap;   // row stride of `rows`
+    int chunks = 1;        // chunks of rows still to arrive (1 when all are here)
     if (!one_trip && width > 0) {
         const size_t need = (size_t)nt * width * sizeof(int);
         if (need > c->h_list_bytes) {
             hfree(c->h_list);
             c->h_list_bytes = 0;
-            HIPCHK(c, hipHostMalloc(&c->h_list, grow(need), hipHostMallocDefault));
+            HIPCHK(c, hipHostMalloc(&c->h_list, grow(need),
+                                    hipHostMallocMapped | hipHostMallocCoherent));
+            void *dev = nullptr;
+            HIPCHK(c, hipHostGetDevicePointer(&dev, c->h_list, 0));
+            c->h_list_dev = static_cast<int *>(dev);
             c->h_list_bytes = grow(need);
         }
-        HIPCHK(c, hipMemcpy2DAsync(c->h_list, (size_t)width * sizeof(int), c->d_list,
-                                   (size_t)cap * sizeof(int), (size_t)width * sizeof(int), nt,
-                                   hipMemcpyDeviceToHost, st));
-        HIPCHK(c, hipStreamSynchronize(st));
         rows = c->h_list;
         stride = width;
+        chunks = (int)std::min<size_t>(std::max<size_t>(1, list_bytes / kFetchChunkBytes),
+                                       std::min<size_t>(abyss_ctx_s::kFetchChunks, nt));
+        for (int k = 0; k < chunks; ++k) {
+            if (!c->fev[k])
+                HIPCHK(c, hipEventCreateWithFlags(&c->fev[k], hipEventDisableTiming));
+            const int q0 = (int)((long long)nt * k / chunks);
+            const int q1 = (int)((long long)nt * (k + 1) / chunks);
+            // another stream than the context's may share the GPU with a
+            // launch that fills it: the copy engine instead of a kernel
+            if (st == c->stream)
+                HIPCHK(c, abyss::launch_pack_rows(c->d_list, c->d_nnb, cap, q0, q1, c->h_list_dev,
+                                                  width, st));
+            else
+                HIPCHK(c, hipMemcpy2DAsync(c->h_list + (size_t)q0 * width,
+                                           (size_t)width * sizeof(int),
+                                           c->d_list + (size_t)q0 * cap,
+                                           (size_t)cap * sizeof(int),
+                                           (size_t)width * sizeof(int), q1 - q0,
+                                           hipMemcpyDeviceToHost, st));
+            HIPCHK(c, hipEventRecord(c->fev[k], st));
+        }
     }
-    memcpy(acc, c->h_res, (size_t)nt * 3 * sizeof(double));
-    memcpy(adot, c->h_res + (size_t)nt * 3, (size_t)nt * 3 * sizeof(double));
-    memcpy(nnb, c->h_nnb, (size_t)nt * sizeof(int));
-    for (int k = 0; k < nt; ++k) {
-        const int cnt = c->h_nnb[k];
-        const int ncopy = std::min(cnt < 0 ? -cnt : cnt, cap);
-        if (ncopy > 0)
-            memcpy(list + (size_t)k * cap, rows + (size_t)k * stride,
-                   (size_t)ncopy * sizeof(int));
-    }
+    const bool arriving = rows == c->h_list && width > 0;
+    hipError_t wait = unpack_results(c, arriving ? chunks : 0, rows, stride, list_bytes, acc, adot,
+                                     nnb, list);
+    HIPCHK(c, wait);
     if (overflowed > 0)
         return set_detail(c, ABYSS_ERR_NEIGHBOR_OVERFLOW,
                           "%d target(s) exceeded the neighbour cap %d", overflowed, cap);
@@ -1118,7 +1268,7 @@ int abyss_ctx_query(abyss_ctx_t c, int nt, const int *targets, double *acc, doub
         return set_detail(c, ABYSS_ERR_INVALID_ARG, "query: null output array");
     int rc = abyss_ctx_set_targets(c, nt, targets);
     if (rc != ABYSS_OK) return rc;
-    rc = abyss_ctx_launch(c);
+    rc = launch_and_keep(c, true);
     if (rc != ABYSS_OK) return rc;
     return abyss_ctx_fetch(c, acc, adot, nnb, list);
 }
@@ -1331,7 +1481,7 @@ int abyss_query_noalloc(int device, int n, const double *jset, int nt, const int
     }
     if (checked)
         NACHK(abyss::launch_recheck_loop(js, fi, counters, nt, rp, rgrid, rpart, fq, acc, adot,
-                                         nullptr, st));
+                                         abyss::FinalMirror{}, nullptr, st));
     if (S == 1) {
         hipLaunchKernelGGL(noalloc_mark_kernel, dim3((nt + 255) / 256), dim3(256), 0, st, targets,
                            nt, n, acc, adot, nnb);

@@ -215,12 +215,24 @@ def error_string(code):
     return load().abyss_error_string(code).decode()
 
 
+def _ref(a, ctype, ptr):
+    """Pointer argument to a C-contiguous array's data.  A reference to its
+    first element costs a sixth of ndarray.ctypes.data_as (which takes what
+    from_buffer does not: read-only and empty arrays)."""
+    if a is None:
+        return None
+    try:
+        return ctypes.byref(ctype.from_buffer(a))
+    except (TypeError, ValueError):
+        return a.ctypes.data_as(ptr)
+
+
 def _d(a):
-    return a.ctypes.data_as(_dp) if a is not None else None
+    return _ref(a, ctypes.c_double, _dp)
 
 
 def _i(a):
-    return a.ctypes.data_as(_ip) if a is not None else None
+    return _ref(a, ctypes.c_int, _ip)
 
 
 def _f64(a, shape=None):

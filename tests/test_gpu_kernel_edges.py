@@ -97,3 +97,34 @@ def test_noalloc_bad_targets_in_every_merge(n, m, prec):
     assert (got[2][bad] == np.iinfo(np.int32).min).all()
     good = np.setdiff1d(np.arange(m), bad)
     assert_same(got, context_query(js, t0, 64, prec), 64, prec, rows=good)
+
+
+@pytest.mark.parametrize("n,m,cap,k_nb", [
+    (1024, 1, 256, 48),        # one split, results written in place
+    (1000, 64, 64, 20),        # the same, the most targets
+    (1500, 65, 64, 20),        # more targets than that
+    (4096, 4096, 30, 40),      # mirrored merge, overflowed lists
+    (20000, 3001, 256, 64),    # mirrored query against a fetch in chunks
+    (20000, 6007, 300, 200),   # several chunks both ways
+    (9000, 4097, 1000, 90)])   # first block above the mirrored ones
+@pytest.mark.parametrize("prec", [regf.PREC_SPLIT, regf.PREC_CHECKED])
+def test_query_equals_launch_and_fetch(n, m, cap, k_nb, prec):
+    """The routes of results to the host give the same bytes and leave the
+    rows past each count alone, also after blocks of other sizes."""
+    say(f"case: results n={n} m={m} cap={cap} precision={prec}")
+    js = workloads.plummer_equal(n, seed=6, k_nb=k_nb)
+    t = np.random.default_rng(m).permutation(n)[:m].astype(np.int32)
+    with regf.Context(device=0, cap=cap, precision=prec) as c:
+        c.upload(js.m, js.x, js.v, js.r2)
+        got = [a.copy() for a in c.query(t)]
+        small = [a.copy() for a in c.query(t[:1])]
+        c.set_targets(t)
+        c.launch()
+        want = c.fetch()
+        again = c.query(t)
+    for a, b, d in zip(got, want, again):
+        assert np.array_equal(a, b) and np.array_equal(a, d)
+    assert small[2][0] == got[2][0] and np.array_equal(small[3][0], got[3][0])
+    filled = np.arange(cap)[None, :] < np.minimum(np.abs(got[2]), cap)[:, None]
+    assert (got[3][~filled] == -1).all() and (got[3][filled] >= 0).all()
+    assert (got[2] < 0).any() == (cap < k_nb)
