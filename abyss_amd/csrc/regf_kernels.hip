@@ -537,6 +537,198 @@ __device__ __forceinline__ void jl_tile_common(JLLane &L, const double2 *__restr
     }
 }
 
+// Four lanes per target on a small j-set (and in FP64 terms on any):
+// neighbours are found and listed in two parts.  A step (or a group of steps)
+// with a neighbour takes a branch that zeroes the near lanes' rsqrt, so that
+// the pair adds exactly 0, and sets the step's bit in a per-lane mask; the
+// masks are listed once per tile, in ascending j.  On a small j-set that
+// branch is not rare: with 100 neighbours per target a group of four steps
+// (256 pairs) holds one with probability 0.9 at N = 10000, 0.6 at N = 30000
+// and 0.1 at N = 262144, and listing each step on its own takes about 25
+// instructions for one or two lanes.  The masks need two more registers,
+// which spill outside the pair loop, so FP32 terms gain up to kMaskedMax
+// particles only.  Force kernel, N / targets, listed per step -> per tile:
+// 10007 / 10007 checked 134 -> 124 us, 16385 / 4096 checked 97 -> 89 us and
+// refined 122 -> 112 us, 30000 / 3000 114 -> 110 us, 30011 / 30011 split even,
+// 262144 / 262144 52.3 -> 52.6 ms; 32 clusters of up to 16384 in a batch
+// 1465 -> 1305 us per launch.  (16 and 64 lanes, whose steps hold fewer
+// targets, lose: N = 2000, every target, 19.5 -> 28.8 us.)
+constexpr int kMaskedMax = 32768;
+struct NearMask {
+    unsigned w0 = 0, w1 = 0;   // steps 0 to 31 and 32 to 63 of the tile
+    __device__ __forceinline__ void set(unsigned bits, int step)
+    {
+        if (step < 32) w0 |= bits << step;
+        else w1 |= bits << (step - 32);
+    }
+};
+
+// Lists a tile's neighbours: bit t of the mask is the lane's pair with
+// record 4 t + sub.  The target itself (by index) and records past `count`
+// (zero-filled) are not listed.
+__device__ __forceinline__ void jl4_list(JLLane &L, NearMask m, int count, int jt)
+{
+    if (L.cap == 0 || !__any((m.w0 | m.w1) != 0)) return;   // cap 0: a recomputation
+    const int j0 = jt + L.sub;                     // the lane's record of step 0
+    const unsigned own = (unsigned)(L.idx - j0);   // 4 t for the target itself
+    if (own < 256u && (own & 3u) == 0) {
+        const unsigned t = own >> 2;
+        if (t < 32) m.w0 &= ~(1u << t);
+        else m.w1 &= ~(1u << (t - 32));
+    }
+    if (count < kTile) {
+        const int valid = (count - L.sub + 3) >> 2;   // steps with a record
+        if (valid < 32) m.w0 &= (1u << max(valid, 0)) - 1u;
+        if (valid < 64) m.w1 &= valid > 32 ? (1u << (valid - 32)) - 1u : 0u;
+    }
+    // the four lanes of a target exchange masks; each lane places its own
+    // neighbours: those of lower steps, and of its step those of the lanes
+    // below it, come first
+    unsigned a[4], b[4];
+    a[0] = __builtin_amdgcn_mov_dpp(m.w0, 0x00, 0xf, 0xf, true);
+    a[1] = __builtin_amdgcn_mov_dpp(m.w0, 0x55, 0xf, 0xf, true);
+    a[2] = __builtin_amdgcn_mov_dpp(m.w0, 0xaa, 0xf, 0xf, true);
+    a[3] = __builtin_amdgcn_mov_dpp(m.w0, 0xff, 0xf, 0xf, true);
+    b[0] = __builtin_amdgcn_mov_dpp(m.w1, 0x00, 0xf, 0xf, true);
+    b[1] = __builtin_amdgcn_mov_dpp(m.w1, 0x55, 0xf, 0xf, true);
+    b[2] = __builtin_amdgcn_mov_dpp(m.w1, 0xaa, 0xf, 0xf, true);
+    b[3] = __builtin_amdgcn_mov_dpp(m.w1, 0xff, 0xf, 0xf, true);
+    const int c0 = L.cnt, c1 = c0 + __popc(a[0]) + __popc(a[1]) + __popc(a[2]) + __popc(a[3]);
+    while (m.w0 | m.w1) {
+        const bool low = m.w0 != 0;
+        const unsigned w = low ? m.w0 : m.w1;
+        const int t = __ffs(w) - 1;
+        if (low) m.w0 = w & (w - 1);
+        else m.w1 = w & (w - 1);
+        const unsigned lt = (1u << t) - 1u, le = 2u * lt + 1u;
+        const int p = (low ? c0 : c1) + __popc((low ? a[0] : b[0]) & (L.sub > 0 ? le : lt)) +
+                      __popc((low ? a[1] : b[1]) & (L.sub > 1 ? le : lt)) +
+                      __popc((low ? a[2] : b[2]) & (L.sub > 2 ? le : lt)) +
+                      __popc((low ? a[3] : b[3]) & lt);
+        if (p < L.cap) L.lst[p] = j0 + 4 * (t + (low ? 0 : 32));
+    }
+    L.cnt = c1 + __popc(b[0]) + __popc(b[1]) + __popc(b[2]) + __popc(b[3]);
+}
+
+// A tile of TILE records for four lanes per target in FP32 terms (TM 0),
+// `count` of them valid (FULL: all; the rest zero-filled, mass 0).  The
+// pairs, the grouped neighbour test and the order of every sum are those of
+// jl_tile_common and jl_tile.
+template <bool FULL, int TILE>
+__device__ __forceinline__ void jl4_tile_fp32(JLLane &L, const double2 *__restrict__ pos,
+                                              const float *__restrict__ mass, int count,
+                                              NearMask &mask)
+{
+    constexpr int JL = 4, G = 4;
+    // whole groups; the records they reach past `count` are in the tile
+    const int steps = FULL ? TILE / JL : (count + JL * G - 1) / (JL * G) * G;
+#pragma unroll 1
+    for (int st = 0; st < steps; st += G) {
+        float dx[G], dy[G], dz[G], rinv[G], dvxg[G], r2[G];
+        float mn = 0.0f;
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const int r = (st + g) * JL + L.sub;
+            const double2 p0 = pos[3 * r + 0];
+            const double2 p1 = pos[3 * r + 1];
+            dx[g] = (float)(p0.x - L.xi);
+            dy[g] = (float)(p0.y - L.yi);
+            dz[g] = (float)(p1.x - L.zi);
+            dvxg[g] = (float)(p1.y - L.vxi);
+            r2[g] = fmaf(dz[g], dz[g], fmaf(dy[g], dy[g], dx[g] * dx[g]));
+            rinv[g] = __builtin_amdgcn_rsqf(r2[g]);
+            mn = g == 0 ? r2[g] : fminf(mn, r2[g]);
+        }
+        if (__any(!(mn > L.rnbf))) {
+            unsigned bits = 0;   // of the group's steps, the first lowest
+#pragma unroll
+            for (int g = G - 1; g >= 0; --g) {
+                const bool near = !(r2[g] > L.rnbf);
+                rinv[g] = near ? 0.0f : rinv[g];
+                bits = 2u * bits + (near ? 1u : 0u);
+            }
+            // volatile: the block stays a branch, not selects for every pair
+            asm volatile("" : "+v"(bits));
+            mask.set(bits, st);
+        }
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const int r = (st + g) * JL + L.sub;
+            const double2 p2 = pos[3 * r + 2];
+            const float mj = mass[r];
+            const float dvx = dvxg[g];
+            const float dvy = (float)(p2.x - L.vyi);
+            const float dvz = (float)(p2.y - L.vzi);
+            const float rinv2 = rinv[g] * rinv[g];
+            const float mr3 = mj * rinv[g] * rinv2;
+            const float rv = fmaf(dz[g], dvz, fmaf(dy[g], dvy, dx[g] * dvx));
+            const float al = -3.0f * rv * rinv2;
+            L.pa[0] = fmaf(mr3, dx[g], L.pa[0]);
+            L.pa[1] = fmaf(mr3, dy[g], L.pa[1]);
+            L.pa[2] = fmaf(mr3, dz[g], L.pa[2]);
+            L.pa[3] = fmaf(mr3, fmaf(al, dx[g], dvx), L.pa[3]);
+            L.pa[4] = fmaf(mr3, fmaf(al, dy[g], dvy), L.pa[4]);
+            L.pa[5] = fmaf(mr3, fmaf(al, dz[g], dvz), L.pa[5]);
+        }
+    }
+}
+
+// The same in FP64 terms (modes 1 to 3): the pairs and sums of jl_tile.
+template <int TM, bool FULL, int TILE>
+__device__ __forceinline__ void jl4_tile_fp64(JLLane &L, const double2 *__restrict__ pos,
+                                              const double *__restrict__ mass, int count,
+                                              NearMask &mask)
+{
+    constexpr int JL = 4;
+    const int steps = FULL ? TILE / JL : (count + JL - 1) / JL;
+    constexpr int kUnroll = FULL ? 2 : 1;   // partial tiles: run-time trip count
+#pragma unroll kUnroll
+    for (int st = 0; st < steps; ++st) {
+        const int r = st * JL + L.sub;
+        const double2 p0 = pos[3 * r + 0];
+        const double2 p1 = pos[3 * r + 1];
+        const double2 p2 = pos[3 * r + 2];
+        const double mj = mass[r];
+        const double dx = p0.x - L.xi;
+        const double dy = p0.y - L.yi;
+        const double dz = p1.x - L.zi;
+        const double dvx = p1.y - L.vxi;
+        const double dvy = p2.x - L.vyi;
+        const double dvz = p2.y - L.vzi;
+        const double r2 = fma(dz, dz, fma(dy, dy, dx * dx));
+        float rf = __builtin_amdgcn_rsqf((float)r2);
+        if (__any(!(r2 > L.rnbd))) {
+            bool near = !(r2 > L.rnbd);
+            if constexpr (TM == 3) {   // mode 0's test, see jl_tile
+                float fx, fy, fz;
+                asm volatile("v_cvt_f32_f64 %0, %1" : "=v"(fx) : "v"(dx));
+                asm volatile("v_cvt_f32_f64 %0, %1" : "=v"(fy) : "v"(dy));
+                asm volatile("v_cvt_f32_f64 %0, %1" : "=v"(fz) : "v"(dz));
+                const float r2f = fmaf(fz, fz, fmaf(fy, fy, fx * fx));
+                near = !(r2f > L.rnbf);
+            }
+            // volatile: a move in the branch, not a select for every pair
+            if (near) asm volatile("v_mov_b32 %0, 0" : "=v"(rf));
+            mask.set(near ? 1u : 0u, st);
+        }
+        double rinv = (double)rf;
+        if constexpr (TM >= 2) {
+            const double h = fma(-(r2 * rinv), rinv, 1.0);
+            rinv = fma(0.5 * rinv, h, rinv);
+        }
+        const double rinv2 = rinv * rinv;
+        const double mr3 = mj * rinv * rinv2;
+        const double rv = fma(dz, dvz, fma(dy, dvy, dx * dvx));
+        const double al = -3.0 * rv * rinv2;
+        L.acc[0] = fma(mr3, dx, L.acc[0]);
+        L.acc[1] = fma(mr3, dy, L.acc[1]);
+        L.acc[2] = fma(mr3, dz, L.acc[2]);
+        L.acc[3] = fma(mr3, fma(al, dx, dvx), L.acc[3]);
+        L.acc[4] = fma(mr3, fma(al, dy, dvy), L.acc[4]);
+        L.acc[5] = fma(mr3, fma(al, dz, dvz), L.acc[5]);
+    }
+}
+
 // EST (mode 0 only): also sum, over the lane's FP32 runs, the squared norms
 // of each run's acceleration and jdot partials, and write the target's two
 // totals to out.spread.  The rounding error of each sum scales with the
@@ -552,13 +744,14 @@ __device__ __forceinline__ void jl_tile_common(JLLane &L, const double2 *__restr
 // split is one tile (the host guarantees jspan <= TILE), loaded at once
 // with TILE / (64 WPB) records per thread into a single LDS buffer, so a
 // split waits for one load instead of one per 256 j.
-template <int JL, int TM, bool EST = false, int TILE = kTile, int WPB = 4>
+template <int JL, int TM, bool EST = false, int TILE = kTile, int WPB = 4, bool MASKED = false>
 __device__ __forceinline__ void regf_body_jl(const JState &js, const int *__restrict__ tgt, int nt,
                                              int jspan, const QueryOut &out, int cap,
                                              int final_counts, int bx, int s, int q_base,
                                              int nt_stride, double2 (*s_pos)[TILE * 3],
                                              typename TermMass<TM>::type (*s_m)[TILE])
 {
+    static_assert(!MASKED || JL == 4, "masks of four lanes per target");
     constexpr bool ONE_SHOT = TILE > 64 * WPB;
     constexpr int R = ONE_SHOT ? TILE / (64 * WPB) : 1;   // records per thread
     static_assert(!ONE_SHOT || TILE % (64 * WPB) == 0, "whole records per thread");
@@ -633,8 +826,19 @@ __device__ __forceinline__ void regf_body_jl(const JState &js, const int *__rest
         if (!ONE_SHOT && t + 1 < ntile && loader) ld.load(js, j0 + (t + 1) * TILE + tid, j1);
         const int jt = j0 + t * TILE;
         const int count = min(TILE, j1 - jt);
+        NearMask near;
         if (!wave_busy) {
             // no target in this wave (the tail of a small block)
+        } else if constexpr (MASKED && TM == 0) {
+            if (count == TILE)
+                jl4_tile_fp32<true, TILE>(L, s_pos[b], s_m[b], count, near);
+            else
+                jl4_tile_fp32<false, TILE>(L, s_pos[b], s_m[b], count, near);
+        } else if constexpr (MASKED) {
+            if (count == TILE)
+                jl4_tile_fp64<TM, true, TILE>(L, s_pos[b], s_m[b], count, near);
+            else
+                jl4_tile_fp64<TM, false, TILE>(L, s_pos[b], s_m[b], count, near);
         } else if (__any((unsigned)(L.idx - jt) < (unsigned)count))
             jl_tile<JL, TM, false, true, TILE>(L, s_pos[b], s_m[b], count, jt);
         else if (count == TILE) {
@@ -660,6 +864,9 @@ __device__ __forceinline__ void regf_body_jl(const JState &js, const int *__rest
             }
         }
         if (!ONE_SHOT && t + 1 < ntile && loader) ld.store(s_pos[b ^ 1], s_m[b ^ 1], tid);
+        // after the wait for the next tile's loads, which would otherwise
+        // wait for these stores as well
+        if constexpr (MASKED) jl4_list(L, near, count, jt);
         __syncthreads();
     }
     double acc[6];
@@ -720,7 +927,7 @@ __device__ __forceinline__ void xcd_place(int id, int total, int gx, int &bx, in
 // A one-shot tile's 52 KB of LDS (56 KB with FP64 masses) holds 3 (2)
 // workgroups per CU, so it asks for 3 (2).
 // Grid: gx * splits workgroups on x (xcd_place).
-template <int JL, int TM, bool EST, int TILE = kTile, int WPB = 4>
+template <int JL, int TM, bool EST, int TILE = kTile, int WPB = 4, bool MASKED = false>
 __global__ __launch_bounds__(64 * WPB)
 __attribute__((amdgpu_waves_per_eu(TILE > 64 * WPB ? (TM == 0 ? 3 : 2) : 5, 8)))
 void regf_kernel_jl(JState js, const int *__restrict__ tgt, int nt, int jspan, QueryOut out,
@@ -733,8 +940,8 @@ void regf_kernel_jl(JState js, const int *__restrict__ tgt, int nt, int jspan, Q
     __shared__ typename TermMass<TM>::type s_m[NB][TILE];
     int bx, s;
     xcd_place(blockIdx.x, gx * splits, gx, bx, s);
-    regf_body_jl<JL, TM, EST, TILE, WPB>(js, tgt, nt, jspan, out, cap, final_counts, bx, s, 0,
-                                         nt, s_pos, s_m);
+    regf_body_jl<JL, TM, EST, TILE, WPB, MASKED>(js, tgt, nt, jspan, out, cap, final_counts, bx,
+                                                 s, 0, nt, s_pos, s_m);
 }
 
 // One wave per target.  Partial sums: lane l adds splits l, l+64, ... in
@@ -1075,7 +1282,7 @@ void recheck_kernel_loop(JState js, const int *__restrict__ tgt, const int *__re
     constexpr int TPB = 4 * (64 / JL);   // targets per workgroup
     const int items = (m + TPB - 1) / TPB * splits;
     for (int it = blockIdx.x; it < items; it += gridDim.x)
-        regf_body_jl<JL, 3>(js, tgt, m, jspan, out, 0, 0, it / splits, it % splits, 0, nt_stride,
+        regf_body_jl<JL, 3, false, kTile, 4, JL == 4>(js, tgt, m, jspan, out, 0, 0, it / splits, it % splits, 0, nt_stride,
                             s_pos, s_m);
 }
 
@@ -1122,7 +1329,7 @@ __device__ __forceinline__ void batch_body(const ClusterDesc &d, const WorkItem 
                                            const QueryOut &out, int cap, int fc,
                                            double2 (*s_pos)[kTile * 3], float (*s_m)[kTile])
 {
-    regf_body_jl<JL, 0, EST, TILE, 4>(d.js, d.tgt, d.nt, d.jspan, out, cap, fc, w.tblock,
+    regf_body_jl<JL, 0, EST, TILE, 4, JL == 4>(d.js, d.tgt, d.nt, d.jspan, out, cap, fc, w.tblock,
                                       w.split, d.q_base, d.nt_stride,
                                       reinterpret_cast<double2 (*)[TILE * 3]>(s_pos),
                                       reinterpret_cast<float (*)[TILE]>(s_m));
@@ -1192,7 +1399,7 @@ void batch_recheck_kernel(const ClusterDesc *__restrict__ cd, const WorkItem *__
         const ClusterDesc &d = cd[w.cluster];
         switch (d.jl) {
             case 4:
-                regf_body_jl<4, 3>(d.js, d.tgt, d.nt, d.jspan, d.part, 0, 0, w.tblock, w.split, 0,
+                regf_body_jl<4, 3, false, kTile, 4, true>(d.js, d.tgt, d.nt, d.jspan, d.part, 0, 0, w.tblock, w.split, 0,
                                    d.nt, s_pos, s_m);
                 break;
             case 16:
@@ -1320,6 +1527,14 @@ template <int JL, bool EST, int TILE, int WPB>
 void launch_shape(const JState &js, const int *tgt, int nt, const Plan &p, const QueryOut &out,
                   int cap, int fc, int *reset, hipStream_t st)
 {
+    if constexpr (JL == 4) {
+        if (js.n <= kMaskedMax) {
+            hipLaunchKernelGGL((regf_kernel_jl<JL, 0, EST, TILE, WPB, true>),
+                               dim3(p.grid_x * p.splits), dim3(64 * WPB), 0, st, js, tgt, nt,
+                               p.jspan, out, cap, fc, reset, p.grid_x, p.splits);
+            return;
+        }
+    }
     hipLaunchKernelGGL((regf_kernel_jl<JL, 0, EST, TILE, WPB>), dim3(p.grid_x * p.splits),
                        dim3(64 * WPB), 0, st, js, tgt, nt, p.jspan, out, cap, fc, reset, p.grid_x,
                        p.splits);
@@ -1375,13 +1590,13 @@ hipError_t launch_jl(const JState &js, const int *tgt, int nt, const Plan &p, co
     else if (tm == 0)
         return launch_mode0<JL, false>(js, tgt, nt, p, out, cap, fc, reset, st);
     else if (tm == 1)
-        hipLaunchKernelGGL((regf_kernel_jl<JL, 1, false>), grid, dim3(kBlock), 0, st, js, tgt,
+        hipLaunchKernelGGL((regf_kernel_jl<JL, 1, false, kTile, 4, JL == 4>), grid, dim3(kBlock), 0, st, js, tgt,
                            nt, p.jspan, out, cap, fc, reset, p.grid_x, p.splits);
     else if (tm == 2)
-        hipLaunchKernelGGL((regf_kernel_jl<JL, 2, false>), grid, dim3(kBlock), 0, st, js, tgt,
+        hipLaunchKernelGGL((regf_kernel_jl<JL, 2, false, kTile, 4, JL == 4>), grid, dim3(kBlock), 0, st, js, tgt,
                            nt, p.jspan, out, cap, fc, reset, p.grid_x, p.splits);
     else
-        hipLaunchKernelGGL((regf_kernel_jl<JL, 3, false>), grid, dim3(kBlock), 0, st, js, tgt,
+        hipLaunchKernelGGL((regf_kernel_jl<JL, 3, false, kTile, 4, JL == 4>), grid, dim3(kBlock), 0, st, js, tgt,
                            nt, p.jspan, out, cap, fc, reset, p.grid_x, p.splits);
     return hipGetLastError();
 }

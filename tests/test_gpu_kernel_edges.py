@@ -128,3 +128,34 @@ def test_query_equals_launch_and_fetch(n, m, cap, k_nb, prec):
     filled = np.arange(cap)[None, :] < np.minimum(np.abs(got[2]), cap)[:, None]
     assert (got[3][~filled] == -1).all() and (got[3][filled] >= 0).all()
     assert (got[2] < 0).any() == (cap < k_nb)
+
+
+@pytest.mark.parametrize("prec", [regf.PREC_SPLIT, regf.PREC_MIXED, regf.PREC_REFINED])
+@pytest.mark.parametrize("n,cap,k_nb,splits", [
+    (5, 8, 3, 1), (256, 64, 40, 1), (257, 64, 40, 1), (1000, 20, 40, 1), (1279, 64, 40, 3),
+    (4099, 400, 350, 2), (32768, 64, 40, 7), (32769, 64, 40, 7)])
+def test_lists_by_tile_equal_lists_by_step(n, cap, k_nb, splits, prec):
+    """Four lanes per target list a tile at a time (up to 32768 particles, and
+    in FP64 terms on any), sixteen a step at a time: the same lists, with own
+    targets, partial tiles, overflow and coincident particles in the way."""
+    say(f"case: lists n={n} cap={cap} splits={splits} precision={prec}")
+    js = workloads.plummer_kroupa(n, seed=8, k_nb=min(k_nb, n - 2))
+    x = js.x.copy()
+    x[n // 2] = x[0]
+    t = np.random.default_rng(n).permutation(n)[:min(n, 2000)].astype(np.int32)
+    out = []
+    with regf.Context(device=0, cap=cap, precision=prec) as c:
+        c.upload(js.m, x, js.v, js.r2)
+        for lanes in (4, 16):
+            c.set_tuning(0, splits, 0, lanes)
+            out.append([a.copy() for a in c.query(t)])
+            assert c.plan()["lanes_per_target"] == lanes
+    a, b = out
+    assert np.array_equal(a[2], b[2]) and np.array_equal(a[3], b[3])
+    assert (np.abs(a[2]) > 0).any()
+    # sums: FP64 terms differ by the order of n additions (n * 2^-53 of the
+    # largest partial, at most 1e4 times the sum), FP32 runs by the rounding
+    # of their 64 terms (64 * 2^-24), both of the whole array
+    tol = 1e-10 if prec != regf.PREC_SPLIT else 4e-6
+    for p, q in zip(a[:2], b[:2]):
+        assert np.linalg.norm(p - q) <= tol * np.linalg.norm(q)
