@@ -72,8 +72,10 @@ struct abyss_ctx_s {
     char *d_rlists = nullptr;
     size_t rlist_bytes = 0;
     int rlist_n = 0;
-    char *d_irr = nullptr, *h_irr = nullptr;  // targets + [nt][6] results
-    size_t irr_bytes = 0;
+    // inputs and results of the list kernels: device copy of the inputs, and
+    // mapped pinned staging (device address h_irr_dev) of both
+    char *d_irr = nullptr, *h_irr = nullptr, *h_irr_dev = nullptr;
+    size_t d_irr_bytes = 0, irr_bytes = 0;
     // 64-byte AoS copy of the j-set {x,y,z,vx,vy,vz,m,0} for the list
     // gathers (one cache line per neighbour instead of seven); rebuilt when
     // jset_version (bumped by every upload / predict) has moved on
@@ -132,6 +134,17 @@ struct abyss_ctx_s {
 
 
 namespace abyss {
+// 64-byte AoS record of the j-set for the list gathers.
+struct __align__(64) JRec {
+    double x, y, z, vx, vy, vz, m, pad;
+};
+// Up to this many targets the list kernels read their targets (and a regular
+// step its dt and a_old) from mapped host memory instead of a device copy: a
+// copy is 3 us before the kernel can start (N = 65536, one target: 19.1 us
+// with it, 16.2 without), but in place every workgroup's 16 bytes are a read
+// over the link of their own; at 16384 targets the two are even (72 to 75 us).
+constexpr int kMappedListTargets = 16384;
+
 // Creates a context that issues all its work on `stream` (owned by the
 // caller) instead of a stream of its own.
 int ctx_create_on_stream(int device, int cap, hipStream_t stream, abyss_ctx_t *out);

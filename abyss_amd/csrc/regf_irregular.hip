@@ -21,6 +21,8 @@
 
 #include <algorithm>
 
+using abyss::JRec;
+
 namespace {
 
 __global__ __launch_bounds__(256) void fill_int_kernel(int *__restrict__ p, size_t count, int v)
@@ -66,10 +68,6 @@ __global__ __launch_bounds__(256) void keep_lists_kernel(const int *__restrict__
     for (int e = lane; e < n; e += 64) rlist[(size_t)i * cap + e] = list[(size_t)q * cap + e];
     if (lane == 0) rnnb[i] = c;
 }
-
-struct __align__(64) JRec {
-    double x, y, z, vx, vy, vz, m, pad;
-};
 
 __global__ __launch_bounds__(256) void pack_aos_kernel(abyss::JState js, int n,
                                                        JRec *__restrict__ out)
@@ -138,29 +136,46 @@ __device__ __forceinline__ int list_len(int c, int cap)
     return min(c < 0 ? -c : c, cap);
 }
 
+// One wave per target.  The four targets of a workgroup put their sums into
+// LDS, from where they go out as two runs of 12 doubles: acc and adot are
+// mapped host memory, to which a wave's own three doubles would be a transfer
+// each.  Bound by the gathers (a 64-byte record per neighbour).
 __global__ __launch_bounds__(256) void irregular_kernel(const JRec *__restrict__ jr,
                                                         const int *__restrict__ tgt, int nt,
                                                         const int *__restrict__ rnnb,
                                                         const int *__restrict__ rlist, int cap,
-                                                        double *__restrict__ out)
+                                                        double *__restrict__ acc,
+                                                        double *__restrict__ adot)
 {
+    __shared__ double s_out[2][12];
     const int lane = threadIdx.x & 63;
-    const int q = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (q >= nt) return;   // wave-uniform; no barriers below
-    const int i = tgt[q];
-    const int n = list_len(rnnb[i], cap);
-    const JRec ri = jr[i];
-    const double xi[3] = {ri.x, ri.y, ri.z};
-    const double vi[3] = {ri.vx, ri.vy, ri.vz};
-    double a[6] = {0, 0, 0, 0, 0, 0};
-    for (int e = lane; e < n; e += 64) {
-        double t[6];
-        term(jr, rlist[(size_t)i * cap + e], xi, vi, t);
+    const int w = threadIdx.x >> 6;
+    const int q = blockIdx.x * 4 + w;
+    if (q < nt) {   // wave-uniform
+        const int i = tgt[q];
+        const int n = list_len(rnnb[i], cap);
+        const JRec ri = jr[i];
+        const double xi[3] = {ri.x, ri.y, ri.z};
+        const double vi[3] = {ri.vx, ri.vy, ri.vz};
+        double a[6] = {0, 0, 0, 0, 0, 0};
+        for (int e = lane; e < n; e += 64) {
+            double t[6];
+            term(jr, rlist[(size_t)i * cap + e], xi, vi, t);
 #pragma unroll
-        for (int k = 0; k < 6; ++k) a[k] += t[k];
+            for (int k = 0; k < 6; ++k) a[k] += t[k];
+        }
+        wave_sum<6>(a);
+        if (lane < 3) {
+            s_out[0][w * 3 + lane] = pick(a[0], a[1], a[2], lane);
+            s_out[1][w * 3 + lane] = pick(a[3], a[4], a[5], lane);
+        }
     }
-    wave_sum<6>(a);
-    if (lane < 6) out[(size_t)q * 6 + lane] = a[lane];
+    __syncthreads();
+    const int rows = 3 * min(4, nt - (int)blockIdx.x * 4);
+    if (threadIdx.x < 12 && (int)threadIdx.x < rows)
+        acc[(size_t)blockIdx.x * 12 + threadIdx.x] = s_out[0][threadIdx.x];
+    else if (threadIdx.x >= 64 && threadIdx.x < 76 && (int)threadIdx.x - 64 < rows)
+        adot[(size_t)blockIdx.x * 12 + threadIdx.x - 64] = s_out[1][threadIdx.x - 64];
 }
 
 // Neighbour-set correction and fourth-order regular corrector of one
@@ -186,6 +201,7 @@ __global__ __launch_bounds__(256) void correct_kernel(
     const double *__restrict__ a_old, double *__restrict__ out)
 {
     extern __shared__ int s_lists[];   // STAGED: [4 waves][new cap | old cap]
+    __shared__ double s_row[4][18];    // a target's results, written out in one run
     const int lane = threadIdx.x & 63;
     const int q = blockIdx.x * 4 + (threadIdx.x >> 6);
     const bool active = q < nt;
@@ -204,6 +220,10 @@ __global__ __launch_bounds__(256) void correct_kernel(
         lo = so;
     }
     if (!active) return;   // wave-uniform; no barriers below
+    // dts and a_old may be mapped host memory: asked for before the gathers
+    const int d = min(lane, 2);   // lanes 0 to 2 take a dimension each
+    const double dt = dts[q];
+    const double a0 = a_old[(size_t)q * 6 + d], j0 = a_old[(size_t)q * 6 + 3 + d];
     const JRec ri = jr[i];
     const double xi[3] = {ri.x, ri.y, ri.z};
     const double vi[3] = {ri.vx, ri.vy, ri.vz};
@@ -229,25 +249,27 @@ __global__ __launch_bounds__(256) void correct_kernel(
         }
     }
     wave_sum<12>(a);
+    double *row = s_row[threadIdx.x >> 6];
     if (lane < 3) {
-        // lane d takes dimension d (selects, not a lane-indexed array)
-        const int d = lane;
-        const double dt = dts[q];
-        const double a0 = a_old[(size_t)q * 6 + d], j0 = a_old[(size_t)q * 6 + 3 + d];
+        // selects, not a lane-indexed array
         const double a1 = new_acc[(size_t)q * 3 + d], j1 = new_adot[(size_t)q * 3 + d];
         const double irr = pick(a[0], a[1], a[2], d), irr_dot = pick(a[3], a[4], a[5], d);
         const double tmp = pick(a[6], a[7], a[8], d), tmp_dot = pick(a[9], a[10], a[11], d);
         double corr[4];
         corrector(dt, a0, j0, a1, j1, tmp, tmp_dot, pick(xi[0], xi[1], xi[2], d),
                   pick(vi[0], vi[1], vi[2], d), corr);
-        double *o = out + (size_t)q * 18;
-        o[d] = corr[0];
-        o[3 + d] = corr[1];
-        o[6 + d] = corr[2];
-        o[9 + d] = corr[3];
-        o[12 + d] = irr;
-        o[15 + d] = irr_dot;
+        row[d] = corr[0];
+        row[3 + d] = corr[1];
+        row[6 + d] = corr[2];
+        row[9 + d] = corr[3];
+        row[12 + d] = irr;
+        row[15 + d] = irr_dot;
     }
+    // the wave's own LDS, written above by three of its lanes
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (lane < 18) out[(size_t)q * 18 + lane] = row[lane];
 }
 
 #pragma clang fp contract(on)
@@ -295,21 +317,31 @@ int ensure_aos(abyss_ctx_t c)
     return ABYSS_OK;
 }
 
-// Device + pinned staging of the irregular / corrector entry points (the
-// stream must be idle: the previous contents may still be in flight).
-int ensure_staging(abyss_ctx_t c, size_t need)
+// Mapped pinned staging of `need` bytes and, for `dev` > 0, a device copy of
+// its first `dev` bytes, for the irregular / corrector entry points (the
+// stream must be idle: the previous contents may still be in use).
+int ensure_staging(abyss_ctx_t c, size_t need, size_t dev)
 {
-    if (need <= c->irr_bytes) return ABYSS_OK;
-    if (c->d_irr) (void)hipFree(c->d_irr);
-    if (c->h_irr) (void)hipHostFree(c->h_irr);
-    c->d_irr = nullptr;
-    c->h_irr = nullptr;
-    c->irr_bytes = 0;
-    const size_t cap = need + need / 2 + 4096;
-    if (hipMalloc(&c->d_irr, cap) != hipSuccess ||
-        hipHostMalloc(&c->h_irr, cap, hipHostMallocDefault) != hipSuccess)
-        return ABYSS_ERR_OUT_OF_MEMORY;
-    c->irr_bytes = cap;
+    if (need > c->irr_bytes) {
+        if (c->h_irr) (void)hipHostFree(c->h_irr);
+        c->h_irr = c->h_irr_dev = nullptr;
+        c->irr_bytes = 0;
+        const size_t cap = need + need / 2 + 4096;
+        void *p = nullptr;
+        if (hipHostMalloc(&c->h_irr, cap, hipHostMallocMapped | hipHostMallocCoherent) !=
+            hipSuccess)
+            return ABYSS_ERR_OUT_OF_MEMORY;
+        if (hipHostGetDevicePointer(&p, c->h_irr, 0) != hipSuccess) return ABYSS_ERR_HIP;
+        c->h_irr_dev = static_cast<char *>(p);
+        c->irr_bytes = cap;
+    }
+    if (dev > c->d_irr_bytes) {
+        if (c->d_irr) (void)hipFree(c->d_irr);
+        c->d_irr = nullptr;
+        c->d_irr_bytes = 0;
+        if (hipMalloc(&c->d_irr, dev + dev / 2) != hipSuccess) return ABYSS_ERR_OUT_OF_MEMORY;
+        c->d_irr_bytes = dev + dev / 2;
+    }
     return ABYSS_OK;
 }
 
@@ -373,32 +405,33 @@ int abyss_ctx_irregular(abyss_ctx_t c, int nt, const int *targets, double *acc, 
     int rc = ensure_resident_lists(c);   // a j-set of another size: empty lists
     if (rc != ABYSS_OK) return rc;
     if (hipStreamSynchronize(c->stream) != hipSuccess) return ABYSS_ERR_HIP;
+    // targets in (read in place up to kMappedListTargets), results straight
+    // into the mapped staging: no copy before or after the kernel and no
+    // transposition on the host.  Bound by the latency of launch and link and,
+    // from some 10000 targets on, by the gathers.  N = 131072, 6000 targets:
+    // 59 us with copies, 43 in place; N = 65536, all targets: 295 and 230.
     const size_t tb = (((size_t)nt * sizeof(int)) + 255) & ~size_t(255);
-    rc = ensure_staging(c, tb + (size_t)nt * 6 * sizeof(double));
+    const size_t ob = (size_t)nt * 3 * sizeof(double);
+    const bool mapped = nt <= abyss::kMappedListTargets;
+    rc = ensure_staging(c, tb + 2 * ob, mapped ? 0 : tb);
     if (rc != ABYSS_OK) return rc;
     memcpy(c->h_irr, targets, (size_t)nt * sizeof(int));
-    if (hipMemcpyAsync(c->d_irr, c->h_irr, (size_t)nt * sizeof(int), hipMemcpyHostToDevice,
-                       c->stream) != hipSuccess)
+    if (!mapped && hipMemcpyAsync(c->d_irr, c->h_irr, (size_t)nt * sizeof(int),
+                                  hipMemcpyHostToDevice, c->stream) != hipSuccess)
         return ABYSS_ERR_HIP;
     const int *rnnb = reinterpret_cast<const int *>(c->d_rlists);
     const int *rlist = rnnb + (((size_t)c->n + 63) & ~size_t(63));
-    double *d_out = reinterpret_cast<double *>(c->d_irr + tb);
     rc = ensure_aos(c);
     if (rc != ABYSS_OK) return rc;
     hipLaunchKernelGGL(irregular_kernel, dim3((nt + 3) / 4), dim3(256), 0, c->stream,
                        reinterpret_cast<const JRec *>(c->d_aos),
-                       reinterpret_cast<const int *>(c->d_irr), nt, rnnb, rlist, c->cap, d_out);
-    if (hipGetLastError() != hipSuccess) return ABYSS_ERR_HIP;
-    double *h_out = reinterpret_cast<double *>(c->h_irr + tb);
-    if (hipMemcpyAsync(h_out, d_out, (size_t)nt * 6 * sizeof(double), hipMemcpyDeviceToHost,
-                       c->stream) != hipSuccess ||
-        hipStreamSynchronize(c->stream) != hipSuccess)
+                       reinterpret_cast<const int *>(mapped ? c->h_irr_dev : c->d_irr), nt, rnnb,
+                       rlist, c->cap, reinterpret_cast<double *>(c->h_irr_dev + tb),
+                       reinterpret_cast<double *>(c->h_irr_dev + tb + ob));
+    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(c->stream) != hipSuccess)
         return ABYSS_ERR_HIP;
-    for (int k = 0; k < nt; ++k)
-        for (int d = 0; d < 3; ++d) {
-            acc[3 * k + d] = h_out[6 * (size_t)k + d];
-            adot[3 * k + d] = h_out[6 * (size_t)k + 3 + d];
-        }
+    memcpy(acc, c->h_irr + tb, ob);
+    memcpy(adot, c->h_irr + tb + ob, ob);
     return ABYSS_OK;
 }
 
@@ -434,18 +467,19 @@ int abyss_ctx_regular_step(abyss_ctx_t c, int nt, const int *targets, const doub
     if (hipStreamSynchronize(c->stream) != hipSuccess) return ABYSS_ERR_HIP;
     // staging: dt [nt] | a_old [nt][6] | out [nt][18]
     const size_t in_bytes = (size_t)nt * 7 * sizeof(double);
-    rc = ensure_staging(c, in_bytes + (size_t)nt * 18 * sizeof(double));
+    const bool mapped = nt <= abyss::kMappedListTargets;
+    rc = ensure_staging(c, in_bytes + (size_t)nt * 18 * sizeof(double), mapped ? 0 : in_bytes);
     if (rc != ABYSS_OK) return rc;
     double *h = reinterpret_cast<double *>(c->h_irr);
     memcpy(h, dt, (size_t)nt * sizeof(double));
     memcpy(h + nt, a_old, (size_t)nt * 6 * sizeof(double));
-    if (hipMemcpyAsync(c->d_irr, c->h_irr, in_bytes, hipMemcpyHostToDevice, c->stream) !=
-        hipSuccess)
+    if (!mapped && hipMemcpyAsync(c->d_irr, c->h_irr, in_bytes, hipMemcpyHostToDevice,
+                                  c->stream) != hipSuccess)
         return ABYSS_ERR_HIP;
     rc = abyss::ctx_launch_force(c, true);   // the fetch below
     if (rc != ABYSS_OK) return rc;
-    const double *d_in = reinterpret_cast<const double *>(c->d_irr);
-    double *d_out = reinterpret_cast<double *>(c->d_irr) + (size_t)nt * 7;
+    const double *d_in = reinterpret_cast<const double *>(mapped ? c->h_irr_dev : c->d_irr);
+    double *d_out = reinterpret_cast<double *>(c->h_irr_dev) + (size_t)nt * 7;
     const int *rnnb = reinterpret_cast<const int *>(c->d_rlists);
     const int *rlist = rnnb + (((size_t)c->n + 63) & ~size_t(63));
     rc = ensure_aos(c);
@@ -467,10 +501,7 @@ int abyss_ctx_regular_step(abyss_ctx_t c, int nt, const int *targets, const doub
     // the resident lists become this step's (after the correction read them)
     rc = abyss::keep_launch_lists(c);
     if (rc != ABYSS_OK) return rc;
-    double *h_out = h + (size_t)nt * 7;
-    if (hipMemcpyAsync(h_out, d_out, (size_t)nt * 18 * sizeof(double), hipMemcpyDeviceToHost,
-                       c->stream) != hipSuccess)
-        return ABYSS_ERR_HIP;
+    const double *h_out = h + (size_t)nt * 7;
     rc = abyss_ctx_fetch(c, acc, adot, nnb, list);   // synchronises the stream
     if (rc != ABYSS_OK && rc != ABYSS_ERR_NEIGHBOR_OVERFLOW) return rc;
     memcpy(out, h_out, (size_t)nt * 18 * sizeof(double));

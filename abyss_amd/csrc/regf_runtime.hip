@@ -682,7 +682,7 @@ unsigned long long ctx_device_bytes(abyss_ctx_t c)
 {
     if (!c) return 0;
     return (unsigned long long)c->j_bytes + c->scratch_bytes + c->state_bytes + c->upd_bytes +
-           c->rlist_bytes + c->irr_bytes + c->aos_bytes + c->drv_bytes + c->rad_bytes +
+           c->rlist_bytes + c->d_irr_bytes + c->aos_bytes + c->drv_bytes + c->rad_bytes +
            (unsigned long long)c->t_capacity * (sizeof(int) * 2 + 6 * sizeof(double) +
                                                 (size_t)c->cap * sizeof(int)) + 256;
 }

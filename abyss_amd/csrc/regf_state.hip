@@ -39,12 +39,15 @@ StateView state_view(const double *base, int n)
 
 #pragma clang fp contract(off)
 __global__ __launch_bounds__(256) void predict_kernel(StateView st, int n, double t_new,
-                                                      double *__restrict__ jx, float *__restrict__ m32)
+                                                      double *__restrict__ jx, float *__restrict__ m32,
+                                                      abyss::JRec *__restrict__ aos)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const size_t N = (size_t)n;
     const double h = t_new - st.t[i];
+    double p[6];
+#pragma unroll
     for (int d = 0; d < 3; ++d) {
         const double x = st.x[d * N + i], v = st.v[d * N + i];
         double xp, vp;
@@ -58,10 +61,14 @@ __global__ __launch_bounds__(256) void predict_kernel(StateView st, int n, doubl
         }
         jx[d * N + i] = xp;
         jx[(3 + d) * N + i] = vp;
+        p[d] = xp;
+        p[3 + d] = vp;
     }
-    jx[6 * N + i] = st.m[i];
+    const double m = st.m[i];
+    jx[6 * N + i] = m;
     jx[7 * N + i] = st.r2[i];
-    m32[i] = (float)st.m[i];
+    m32[i] = (float)m;
+    if (aos) aos[i] = abyss::JRec{p[0], p[1], p[2], p[3], p[4], p[5], m, 0.0};
 }
 #pragma clang fp contract(on)
 
@@ -227,10 +234,17 @@ int abyss_ctx_predict(abyss_ctx_t c, double t_new)
     const int n = c->state_n;
     double *jx = reinterpret_cast<double *>(c->d_j);
     float *m32 = reinterpret_cast<float *>(jx + 8 * (size_t)n);
+    // with resident lists in use, their gather records come from the same
+    // pass (a pack of their own otherwise: 5 us at N = 65536)
+    abyss::JRec *aos = c->keep_lists && c->aos_bytes >= (size_t)n * sizeof(abyss::JRec)
+                           ? reinterpret_cast<abyss::JRec *>(c->d_aos)
+                           : nullptr;
     hipLaunchKernelGGL(predict_kernel, dim3((n + 255) / 256), dim3(256), 0, c->stream,
-                       state_view(c->d_state, n), n, t_new, jx, m32);
+                       state_view(c->d_state, n), n, t_new, jx, m32, aos);
     c->jset_version += 1;
-    return hipGetLastError() == hipSuccess ? ABYSS_OK : ABYSS_ERR_HIP;
+    if (hipGetLastError() != hipSuccess) return ABYSS_ERR_HIP;
+    if (aos) c->aos_version = c->jset_version;
+    return ABYSS_OK;
 }
 
 }  // extern "C"

@@ -159,3 +159,43 @@ def test_lists_by_tile_equal_lists_by_step(n, cap, k_nb, splits, prec):
     tol = 1e-10 if prec != regf.PREC_SPLIT else 4e-6
     for p, q in zip(a[:2], b[:2]):
         assert np.linalg.norm(p - q) <= tol * np.linalg.norm(q)
+
+
+@pytest.mark.parametrize("nt", [1, 3, 4, 5, 16384, 16385])
+def test_list_kernels_from_mapped_memory(nt):
+    """Up to 16384 targets the list kernels read their inputs in place and in
+    any case write their results in place, four targets a workgroup: each
+    target's values equal those of a call by 777 others, bit for bit; the
+    gather records written by a prediction equal those packed from a j-set."""
+    say(f"case: list kernels targets={nt}")
+    n, t_new = 20000, 2.0 ** -7
+    js = workloads.plummer_kroupa(n, seed=4, k_nb=40)
+    rng = np.random.default_rng(nt)
+    t = rng.permutation(n)[:nt].astype(np.int32)
+    dt = rng.uniform(1e-3, 1e-2, nt)
+    a_old = rng.normal(size=(nt, 6))
+    parts = [slice(k, min(k + 777, nt)) for k in range(0, nt, 777)]
+    every = np.arange(n, dtype=np.int32)
+    with regf.Context(device=0, cap=200) as c, regf.Context(device=0, cap=200) as d:
+        for k in (c, d):
+            k.upload(js.m, js.x, js.v, js.r2)
+            k.keep_lists()
+            k.query(every)
+        acc, adot = c.irregular(t)
+        for s in parts:
+            p, q = d.irregular(t[s])
+            assert np.array_equal(acc[s], p) and np.array_equal(adot[s], q)
+        # c: records of the prediction; d: records packed from an uploaded j-set
+        z = np.zeros((n, 3))
+        c.upload_state(js.m, js.x, js.v, z, z, np.zeros(n), js.r2)
+        c.predict(t_new)
+        c.query(every)
+        d.upload(js.m, js.x + t_new * js.v, js.v, js.r2)
+        d.query(every)
+        acc, adot = c.irregular(t)
+        out = c.regular_step(t, dt, a_old)[4]
+        for s in parts:
+            p, q = d.irregular(t[s])
+            assert np.array_equal(acc[s], p) and np.array_equal(adot[s], q)
+        for s in parts:
+            assert np.array_equal(out[s][:, 12:], d.regular_step(t[s], dt[s], a_old[s])[4][:, 12:])
