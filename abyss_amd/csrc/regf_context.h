@@ -28,6 +28,15 @@ struct abyss_ctx_s {
     int nt = 0;
     bool counts_valid = false;   // d_nnb holds the counts of the current targets
     size_t t_capacity = 0;  // targets the output buffers can hold
+    // Work on the stream that may not have finished and uses host staging or
+    // the target and output buffers: a target list's way to the device or a
+    // launch (busy_tgt), the list kernels (busy_irr), a state update
+    // (busy_upd).  ctx_wait clears them.  A call that only needs one of these
+    // buffers need not wait for an upload or a prediction before it.
+    bool busy_tgt = false, busy_irr = false, busy_upd = false;
+    // no caller can put work of its own on the stream (the drop-in calls'
+    // context), so the flags tell all there is
+    bool closed = false;
     int *d_tgt = nullptr, *h_tgt = nullptr;
     // h_tgt is mapped, coherent pinned memory; h_tgt_dev is its device
     // address.  `tgt` is the target array the kernels read: h_tgt_dev for
@@ -62,7 +71,7 @@ struct abyss_ctx_s {
     double *d_state = nullptr, *h_state = nullptr;
     size_t state_bytes = 0;
     int state_n = 0;
-    char *d_upd = nullptr, *h_upd = nullptr;
+    char *h_upd = nullptr, *h_upd_dev = nullptr;
     size_t upd_bytes = 0;
 
     // resident neighbour lists (regf_irregular.hip): [nnb: n ints, padded
@@ -163,9 +172,12 @@ int ctx_launch_force(abyss_ctx_t c, bool to_host = false);
 int keep_launch_lists(abyss_ctx_t c);
 // Checked precision: the spread / flag buffers for nt targets and S splits.
 int ctx_ensure_check(abyss_ctx_t c, int nt, int S);
-// abyss_ctx_set_targets with (sync) or without the wait for the context's
-// stream; _idle: the caller guarantees that no launch using this context
-// is in flight (an ensemble member whose last batch has finished).
-int ctx_set_targets_sync(abyss_ctx_t c, int nt, const int *targets, bool sync);
-int ctx_set_targets_idle(abyss_ctx_t c, int nt, const int *targets);
+// abyss_ctx_set_targets that waits for the context's stream always, only for
+// work that uses the target list or the outputs (a synchronous call's own
+// step), or not at all (the caller guarantees that no launch using this
+// context is in flight: an ensemble member whose last batch has finished).
+enum class TargetWait { kStream, kUse, kNone };
+int ctx_set_targets(abyss_ctx_t c, int nt, const int *targets, TargetWait wait);
+// Waits for the context's stream.
+int ctx_wait(abyss_ctx_t c);
 }  // namespace abyss

@@ -435,7 +435,7 @@ int abyss_ens_set_targets(abyss_ens_t e, int cluster, int nt, const int *targets
     // launch has finished; other clusters' launches may still run
     int rc = wait_cluster(e, cluster);
     if (rc != ABYSS_OK) return rc;
-    rc = abyss::ctx_set_targets_idle(c, nt, targets);
+    rc = abyss::ctx_set_targets(c, nt, targets, abyss::TargetWait::kNone);
     e->active[cluster] = rc == ABYSS_OK ? 1 : 0;
     e->chk_done[cluster] = 0;
     e->blk_first[cluster] = 0;

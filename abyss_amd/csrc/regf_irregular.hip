@@ -404,7 +404,7 @@ int abyss_ctx_irregular(abyss_ctx_t c, int nt, const int *targets, double *acc, 
     if (hipSetDevice(c->device) != hipSuccess) return ABYSS_ERR_HIP;
     int rc = ensure_resident_lists(c);   // a j-set of another size: empty lists
     if (rc != ABYSS_OK) return rc;
-    if (hipStreamSynchronize(c->stream) != hipSuccess) return ABYSS_ERR_HIP;
+    if (c->busy_irr && (rc = abyss::ctx_wait(c)) != ABYSS_OK) return rc;
     // targets in (read in place up to kMappedListTargets), results straight
     // into the mapped staging: no copy before or after the kernel and no
     // transposition on the host.  Bound by the latency of launch and link and,
@@ -416,6 +416,7 @@ int abyss_ctx_irregular(abyss_ctx_t c, int nt, const int *targets, double *acc, 
     rc = ensure_staging(c, tb + 2 * ob, mapped ? 0 : tb);
     if (rc != ABYSS_OK) return rc;
     memcpy(c->h_irr, targets, (size_t)nt * sizeof(int));
+    c->busy_irr = true;
     if (!mapped && hipMemcpyAsync(c->d_irr, c->h_irr, (size_t)nt * sizeof(int),
                                   hipMemcpyHostToDevice, c->stream) != hipSuccess)
         return ABYSS_ERR_HIP;
@@ -428,8 +429,9 @@ int abyss_ctx_irregular(abyss_ctx_t c, int nt, const int *targets, double *acc, 
                        reinterpret_cast<const int *>(mapped ? c->h_irr_dev : c->d_irr), nt, rnnb,
                        rlist, c->cap, reinterpret_cast<double *>(c->h_irr_dev + tb),
                        reinterpret_cast<double *>(c->h_irr_dev + tb + ob));
-    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(c->stream) != hipSuccess)
-        return ABYSS_ERR_HIP;
+    if (hipGetLastError() != hipSuccess) return ABYSS_ERR_HIP;
+    rc = abyss::ctx_wait(c);
+    if (rc != ABYSS_OK) return rc;
     memcpy(acc, c->h_irr + tb, ob);
     memcpy(adot, c->h_irr + tb + ob, ob);
     return ABYSS_OK;
@@ -459,12 +461,13 @@ int abyss_ctx_regular_step(abyss_ctx_t c, int nt, const int *targets, const doub
                 return ABYSS_ERR_INVALID_INPUT;
             }
     }
-    int rc = abyss_ctx_set_targets(c, nt, targets);   // validates the targets
+    // validates the targets
+    int rc = abyss::ctx_set_targets(c, nt, targets, abyss::TargetWait::kUse);
     if (rc != ABYSS_OK) return rc;
     if (hipSetDevice(c->device) != hipSuccess) return ABYSS_ERR_HIP;
     rc = ensure_resident_lists(c);
     if (rc != ABYSS_OK) return rc;
-    if (hipStreamSynchronize(c->stream) != hipSuccess) return ABYSS_ERR_HIP;
+    if (c->busy_irr && (rc = abyss::ctx_wait(c)) != ABYSS_OK) return rc;
     // staging: dt [nt] | a_old [nt][6] | out [nt][18]
     const size_t in_bytes = (size_t)nt * 7 * sizeof(double);
     const bool mapped = nt <= abyss::kMappedListTargets;
@@ -473,6 +476,7 @@ int abyss_ctx_regular_step(abyss_ctx_t c, int nt, const int *targets, const doub
     double *h = reinterpret_cast<double *>(c->h_irr);
     memcpy(h, dt, (size_t)nt * sizeof(double));
     memcpy(h + nt, a_old, (size_t)nt * 6 * sizeof(double));
+    c->busy_irr = true;
     if (!mapped && hipMemcpyAsync(c->d_irr, c->h_irr, in_bytes, hipMemcpyHostToDevice,
                                   c->stream) != hipSuccess)
         return ABYSS_ERR_HIP;

@@ -73,6 +73,7 @@ int legacy_init(int irank)
         return rc;
     }
     g_init_detail[0] = 0;
+    g_ctx->closed = true;
     abyss_ctx_set_precision(g_ctx, g_prec);
     return ABYSS_OK;
 }

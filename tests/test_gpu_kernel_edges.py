@@ -199,3 +199,38 @@ def test_list_kernels_from_mapped_memory(nt):
             assert np.array_equal(acc[s], p) and np.array_equal(adot[s], q)
         for s in parts:
             assert np.array_equal(out[s][:, 12:], d.regular_step(t[s], dt[s], a_old[s])[4][:, 12:])
+
+
+@pytest.mark.parametrize("count", [1, 63, 64, 65, 1500])
+def test_updates_and_calls_that_do_not_wait(count):
+    """Records that reach the state by way of LDS, two updates one after the
+    other, and steps queued behind an update and a prediction: the same bytes
+    as from a j-set uploaded at once."""
+    say(f"case: updates count={count}")
+    n, t_new, cap = 3000, 2.0 ** -6, 150
+    js = workloads.plummer_kroupa(n, seed=12, k_nb=30)
+    rng = np.random.default_rng(count)
+    m, x, v, r2 = js.m.copy(), js.x.copy(), js.v.copy(), js.r2.copy()
+    zero = np.zeros((n, 3))
+    with regf.Context(device=0, cap=cap) as c, regf.Context(device=0, cap=cap) as d:
+        c.upload_state(m, x, v, zero, zero, np.zeros(n), r2)
+        c.keep_lists()
+        for nt in (70, 3, 64, 65, 900, n, 1, 300):
+            for _ in range(2):
+                i = rng.permutation(n)[:count].astype(np.int32)
+                x[i] += 1e-3 * rng.normal(size=(count, 3))
+                v[i] *= 1.01
+                m[i] *= 0.99
+                r2[i] *= 1.02
+                z = zero[:count]
+                c.update_state(i, m[i], x[i], v[i], z, z, np.zeros(count), r2[i])
+            c.predict(t_new)
+            t = rng.permutation(n)[:nt].astype(np.int32)
+            if nt % 2:
+                got = c.regular_step(t, np.full(nt, 1e-3), np.zeros((nt, 6)))[:4]
+            else:
+                got = c.query(t)
+            d.upload(m, x + t_new * v, v, r2)
+            want = d.query(t)
+            for p, q in zip(got, want):
+                assert np.array_equal(p, q)
