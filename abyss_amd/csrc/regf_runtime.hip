@@ -917,9 +917,13 @@ int ctx_set_targets(abyss_ctx_t c, int nt, const int *targets, TargetWait wait)
     if (rc != ABYSS_OK) return rc;
     memcpy(c->h_tgt, targets, (size_t)nt * sizeof(int));
     c->busy_tgt = true;   // until the stream is next waited for
-    if (nt <= kMappedTargets && !c->batch_member) {
+    if (nt <= kMappedTargets || c->batch_member) {
         // small block: kernels read the (coherent) pinned copy directly; no
-        // launch still reads the previous list
+        // launch still reads the previous list.  A batch member's list also:
+        // its 256 bytes per work item cost nothing next to the item, a copy
+        // for every cluster 3 us of the calling thread (32 clusters 178 -> 87
+        // us).  (For other blocks the two are even: 1000 targets 136 us, 4096
+        // 354 to 360.)
         c->tgt = c->h_tgt_dev;
     } else {
         HIPCHK(c, hipMemcpyAsync(c->d_tgt, c->h_tgt, (size_t)nt * sizeof(int),
