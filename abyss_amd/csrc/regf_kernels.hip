@@ -470,7 +470,13 @@ __device__ __forceinline__ void jl_tile(JLLane &L, const double2 *__restrict__ p
 // rsqrt; the rare branch recomputes r^2 from the same differences with the
 // same expression, hence the same bits.  That keeps the group's state at 5
 // registers per step.
-template <int JL, int G, int TILE>
+// PRIO: a wave in the test and terms of a group goes before the waves that are
+// still forming differences, so that the phases of a SIMD's waves drift apart
+// and the FP64 differences of some issue between the FP32 terms of others.
+// King N = 262144, every target: force kernel 52.6 -> 52.1 ms; 30011 split 874
+// -> 863 us; N = 65536, 20011 targets 1188 -> 1178 us.  With few tiles per
+// workgroup it costs: N = 65536, 1000 targets (2 tiles) 80 -> 84 us.
+template <int JL, int G, int TILE, bool PRIO>
 __device__ __forceinline__ void jl_tile_common(JLLane &L, const double2 *__restrict__ pos,
                                                const float *__restrict__ mass, int jt)
 {
@@ -478,6 +484,7 @@ __device__ __forceinline__ void jl_tile_common(JLLane &L, const double2 *__restr
     static_assert(steps % G == 0, "the group divides the tile");
 #pragma unroll 1
     for (int st = 0; st < steps; st += G) {
+        if constexpr (PRIO) __builtin_amdgcn_s_setprio(0);
         float dx[G], dy[G], dz[G], rinv[G], dvxg[G];
         float mn = 0.0f;
 #pragma unroll
@@ -493,6 +500,7 @@ __device__ __forceinline__ void jl_tile_common(JLLane &L, const double2 *__restr
             rinv[g] = __builtin_amdgcn_rsqf(r2);
             mn = g == 0 ? r2 : fminf(mn, r2);
         }
+        if constexpr (PRIO) __builtin_amdgcn_s_setprio(1);
         if (__any(!(mn > L.rnbf))) {
 #pragma unroll
             for (int g = 0; g < G; ++g) {
@@ -554,6 +562,9 @@ __device__ __forceinline__ void jl_tile_common(JLLane &L, const double2 *__restr
 // 1465 -> 1305 us per launch.  (16 and 64 lanes, whose steps hold fewer
 // targets, lose: N = 2000, every target, 19.5 -> 28.8 us.)
 constexpr int kMaskedMax = 32768;
+// Four lanes per target in FP32 terms above that: waves take priorities (PRIO
+// of jl_tile_common) from this span on.
+constexpr int kPrioSpan = 8 * kTile;
 struct NearMask {
     unsigned w0 = 0, w1 = 0;   // steps 0 to 31 and 32 to 63 of the tile
     __device__ __forceinline__ void set(unsigned bits, int step)
@@ -624,6 +635,7 @@ __device__ __forceinline__ void jl4_tile_fp32(JLLane &L, const double2 *__restri
     const int steps = FULL ? TILE / JL : (count + JL * G - 1) / (JL * G) * G;
 #pragma unroll 1
     for (int st = 0; st < steps; st += G) {
+        __builtin_amdgcn_s_setprio(0);   // as PRIO of jl_tile_common
         float dx[G], dy[G], dz[G], rinv[G], dvxg[G], r2[G];
         float mn = 0.0f;
 #pragma unroll
@@ -639,6 +651,7 @@ __device__ __forceinline__ void jl4_tile_fp32(JLLane &L, const double2 *__restri
             rinv[g] = __builtin_amdgcn_rsqf(r2[g]);
             mn = g == 0 ? r2[g] : fminf(mn, r2[g]);
         }
+        __builtin_amdgcn_s_setprio(1);
         if (__any(!(mn > L.rnbf))) {
             unsigned bits = 0;   // of the group's steps, the first lowest
 #pragma unroll
@@ -744,7 +757,8 @@ __device__ __forceinline__ void jl4_tile_fp64(JLLane &L, const double2 *__restri
 // split is one tile (the host guarantees jspan <= TILE), loaded at once
 // with TILE / (64 WPB) records per thread into a single LDS buffer, so a
 // split waits for one load instead of one per 256 j.
-template <int JL, int TM, bool EST = false, int TILE = kTile, int WPB = 4, bool MASKED = false>
+template <int JL, int TM, bool EST = false, int TILE = kTile, int WPB = 4, bool MASKED = false,
+          bool PRIO = JL == 16>
 __device__ __forceinline__ void regf_body_jl(const JState &js, const int *__restrict__ tgt, int nt,
                                              int jspan, const QueryOut &out, int cap,
                                              int final_counts, int bx, int s, int q_base,
@@ -843,7 +857,7 @@ __device__ __forceinline__ void regf_body_jl(const JState &js, const int *__rest
             jl_tile<JL, TM, false, true, TILE>(L, s_pos[b], s_m[b], count, jt);
         else if (count == TILE) {
             if constexpr (TM == 0)
-                jl_tile_common<JL, G, TILE>(L, s_pos[b], s_m[b], jt);
+                jl_tile_common<JL, G, TILE, PRIO>(L, s_pos[b], s_m[b], jt);
             else
                 jl_tile<JL, TM, true, false, TILE>(L, s_pos[b], s_m[b], count, jt);
         }
@@ -927,7 +941,8 @@ __device__ __forceinline__ void xcd_place(int id, int total, int gx, int &bx, in
 // A one-shot tile's 52 KB of LDS (56 KB with FP64 masses) holds 3 (2)
 // workgroups per CU, so it asks for 3 (2).
 // Grid: gx * splits workgroups on x (xcd_place).
-template <int JL, int TM, bool EST, int TILE = kTile, int WPB = 4, bool MASKED = false>
+template <int JL, int TM, bool EST, int TILE = kTile, int WPB = 4, bool MASKED = false,
+          bool PRIO = JL == 16>
 __global__ __launch_bounds__(64 * WPB)
 __attribute__((amdgpu_waves_per_eu(TILE > 64 * WPB ? (TM == 0 ? 3 : 2) : 5, 8)))
 void regf_kernel_jl(JState js, const int *__restrict__ tgt, int nt, int jspan, QueryOut out,
@@ -940,8 +955,8 @@ void regf_kernel_jl(JState js, const int *__restrict__ tgt, int nt, int jspan, Q
     __shared__ typename TermMass<TM>::type s_m[NB][TILE];
     int bx, s;
     xcd_place(blockIdx.x, gx * splits, gx, bx, s);
-    regf_body_jl<JL, TM, EST, TILE, WPB, MASKED>(js, tgt, nt, jspan, out, cap, final_counts, bx,
-                                                 s, 0, nt, s_pos, s_m);
+    regf_body_jl<JL, TM, EST, TILE, WPB, MASKED, PRIO>(js, tgt, nt, jspan, out, cap, final_counts,
+                                                       bx, s, 0, nt, s_pos, s_m);
 }
 
 // One wave per target.  Partial sums: lane l adds splits l, l+64, ... in
@@ -1533,6 +1548,14 @@ void launch_shape(const JState &js, const int *tgt, int nt, const Plan &p, const
                                dim3(p.grid_x * p.splits), dim3(64 * WPB), 0, st, js, tgt, nt,
                                p.jspan, out, cap, fc, reset, p.grid_x, p.splits);
             return;
+        }
+        if constexpr (TILE == kTile && WPB == 4) {
+            if (p.jspan >= kPrioSpan) {
+                hipLaunchKernelGGL((regf_kernel_jl<JL, 0, EST, TILE, WPB, false, true>),
+                                   dim3(p.grid_x * p.splits), dim3(64 * WPB), 0, st, js, tgt, nt,
+                                   p.jspan, out, cap, fc, reset, p.grid_x, p.splits);
+                return;
+            }
         }
     }
     hipLaunchKernelGGL((regf_kernel_jl<JL, 0, EST, TILE, WPB>), dim3(p.grid_x * p.splits),
