@@ -65,6 +65,13 @@ struct abyss_ctx_s {
     // one event per chunk of a large fetch
     static constexpr int kFetchChunks = 16;
     hipEvent_t fev[kFetchChunks] = {};
+    // list rows under way on `side`, beside the recomputation of checked
+    // precision, to the fetch that follows the launch (set by the launch)
+    hipStream_t side = nullptr;
+    hipEvent_t sums_ev = nullptr;
+    bool rows_sent = false, side_busy = false;
+    int rows_chunks = 0, rows_width = 0, rows_overflowed = 0;
+    size_t rows_bytes = 0;
 
     // device-resident particle state (regf_state.hip): SoA x,v,a,adot (3n
     // each), t, m, r2 (n each); staging for incremental updates

@@ -212,9 +212,10 @@ hipError_t launch_finalize(const QueryOut &part, int S, int nt, int cap,
                            const TargetGuard &guard = TargetGuard{});
 
 // Copies the populated entries of list rows [q0, q1) (row stride cap) to
-// `rows` (mapped host memory, row stride `width` >= every populated count).
+// `rows` (mapped host memory, row stride `width` >= every populated count) with
+// at most `groups` workgroups.
 hipError_t launch_pack_rows(const int *list, const int *nnb, int cap, int q0, int q1, int *rows,
-                            int width, hipStream_t st);
+                            int width, int groups, hipStream_t st);
 
 // Checked precision.  counters[0] must be 0.  Appends to (fq, fi) the
 // position and j-index of every target q whose a or jdot may be off by

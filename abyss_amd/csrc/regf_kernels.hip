@@ -1239,12 +1239,12 @@ __global__ __launch_bounds__(256) void pack_rows_kernel(const int *__restrict__ 
                                                         int width)
 {
     const int lane = threadIdx.x & 63;
-    const int q = q0 + blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (q >= q1) return;   // the whole wave
-    const int c = nnb[q];
-    const int n = min(min(c < 0 ? -c : c, cap), width);
-    for (int e = lane; e < n; e += 64)
-        rows[(size_t)q * width + e] = list[(size_t)q * cap + e];
+    for (int q = q0 + blockIdx.x * 4 + (threadIdx.x >> 6); q < q1; q += gridDim.x * 4) {
+        const int c = nnb[q];
+        const int n = min(min(c < 0 ? -c : c, cap), width);
+        for (int e = lane; e < n; e += 64)
+            rows[(size_t)q * width + e] = list[(size_t)q * cap + e];
+    }
 }
 
 // ---- checked precision ---------------------------------------------------
@@ -1721,11 +1721,12 @@ hipError_t launch_check_flag(const double *acc, const double *adot, const float 
 }
 
 hipError_t launch_pack_rows(const int *list, const int *nnb, int cap, int q0, int q1, int *rows,
-                            int width, hipStream_t st)
+                            int width, int groups, hipStream_t st)
 {
     if (q1 <= q0) return hipSuccess;
-    hipLaunchKernelGGL(pack_rows_kernel, dim3((q1 - q0 + 3) / 4), dim3(256), 0, st, list, nnb, cap,
-                       q0, q1, rows, width);
+    if (groups <= 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(pack_rows_kernel, dim3(std::min((q1 - q0 + 3) / 4, groups)), dim3(256), 0,
+                       st, list, nnb, cap, q0, q1, rows, width);
     return hipGetLastError();
 }
 

@@ -56,6 +56,12 @@ constexpr size_t kQueryMirrorRowBytes = 4u << 20;
 constexpr size_t kFetchChunkBytes = 2u << 20;
 constexpr size_t kUnpackParallelBytes = 1u << 20;
 constexpr int kUnpackParts = 8;
+// Workgroups of the kernel that sends list rows beside the recomputation: the
+// link takes no more than these store, and every one of them takes a place
+// from the recomputation.  King N = 262144, every target, query: 16 workgroups
+// 60.2 ms, 64 56.7, 256 56.6, one per four rows 57.3; N = 65536, 20011 targets
+// 1633, 1440, 1441, 1421 us.
+constexpr int kPackGroupsBeside = 256;
 // Most j-splits of the recomputation that reads its count on the device
 // (scratch: this many rows per target of the block, 52 bytes each).
 constexpr int kRecheckLoopSplits = 256;
@@ -483,6 +489,60 @@ int ensure_recheck_scratch(abyss_ctx_t c, size_t rows, QueryOut *rpart)
     return ABYSS_OK;
 }
 
+// With the counts in h_nnb, enqueues on `st` the populated entries of the list
+// rows, to h_list at the stride that fits the longest, in chunks; chunk k has
+// arrived once c->fev[k] has completed.  By a kernel of at most `groups`
+// workgroups; 0: by the copy engine.
+int send_rows(abyss_ctx_t c, hipStream_t st, int groups)
+{
+    const int nt = c->nt, cap = c->cap;
+    int width = 0, overflowed = 0;
+    size_t entries = 0;
+    for (int k = 0; k < nt; ++k) {
+        const int cnt = c->h_nnb[k];
+        const int n = std::min(cnt < 0 ? -cnt : cnt, cap);
+        width = std::max(width, n);
+        overflowed += cnt < 0;
+        entries += n;
+    }
+    c->rows_width = width;
+    c->rows_overflowed = overflowed;
+    c->rows_bytes = entries * sizeof(int);
+    c->rows_chunks = 0;
+    if (width == 0) return ABYSS_OK;
+    const size_t need = (size_t)nt * width * sizeof(int);
+    if (need > c->h_list_bytes) {
+        hfree(c->h_list);
+        c->h_list_bytes = 0;
+        HIPCHK(c, hipHostMalloc(&c->h_list, grow(need),
+                                hipHostMallocMapped | hipHostMallocCoherent));
+        void *dev = nullptr;
+        HIPCHK(c, hipHostGetDevicePointer(&dev, c->h_list, 0));
+        c->h_list_dev = static_cast<int *>(dev);
+        c->h_list_bytes = grow(need);
+    }
+    const int chunks = (int)std::min<size_t>(
+        std::max<size_t>(1, c->rows_bytes / kFetchChunkBytes),
+        std::min<size_t>(abyss_ctx_s::kFetchChunks, nt));
+    for (int k = 0; k < chunks; ++k) {
+        if (!c->fev[k]) HIPCHK(c, hipEventCreateWithFlags(&c->fev[k], hipEventDisableTiming));
+        const int q0 = (int)((long long)nt * k / chunks);
+        const int q1 = (int)((long long)nt * (k + 1) / chunks);
+        if (groups > 0)
+            HIPCHK(c, abyss::launch_pack_rows(c->d_list, c->d_nnb, cap, q0, q1, c->h_list_dev,
+                                              width, groups, st));
+        else
+            HIPCHK(c, hipMemcpy2DAsync(c->h_list + (size_t)q0 * width,
+                                       (size_t)width * sizeof(int),
+                                       c->d_list + (size_t)q0 * cap, (size_t)cap * sizeof(int),
+                                       (size_t)width * sizeof(int), q1 - q0,
+                                       hipMemcpyDeviceToHost, st));
+        HIPCHK(c, hipEventRecord(c->fev[k], st));
+    }
+    c->rows_chunks = chunks;
+    return ABYSS_OK;
+}
+
 // The recomputation of m flagged targets (c->chk_fq / chk_fi hold them),
 // planned for m; the stream need not be idle.
 int recompute_flagged(abyss_ctx_t c, int m, const abyss::FinalMirror &mirror)
@@ -531,8 +591,12 @@ Plan plan_recheck_loop(abyss_ctx_t c, int nt, int n, int max_splits, int *grid)
 // same regular set: the flagged count is read back (a host wait) and the
 // recomputation planned for it.  (Blocks small enough to skip that wait run
 // in FP64 terms in one pass instead, Plan::fp64_terms.)  The recomputed
-// targets' results also go to the mirror when it is set.
-int recheck(abyss_ctx_t c, bool flagged, const abyss::FinalMirror &mirror)
+// targets' results also go to the mirror when it is set.  rows_early: a fetch
+// follows, and the list rows, which the recomputation leaves as they are,
+// start on their way to the host beside it.  King N = 262144, every target
+// (recomputation 4.9 ms, rows 2.2 ms): query 60.1 -> 56.6 ms; N = 65536, 20011
+// targets 1455 -> 1441 us.
+int recheck(abyss_ctx_t c, bool flagged, const abyss::FinalMirror &mirror, bool rows_early)
 {
     if (!flagged) {
         // one-split launches: a flag pass over the final results (the force
@@ -561,7 +625,20 @@ int recheck(abyss_ctx_t c, bool flagged, const abyss::FinalMirror &mirror)
     HIPCHK(c, hipMemcpyAsync(c->h_chk, c->chk_counters, sizeof(int), hipMemcpyDeviceToHost,
                              c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    return recompute_flagged(c, c->h_chk[0], mirror);
+    int rc = recompute_flagged(c, c->h_chk[0], mirror);
+    if (rc != ABYSS_OK || !rows_early) return rc;
+    // the merge has finished, so the side stream need not wait for it
+    rc = ensure_host_rows(c, 0);
+    if (rc != ABYSS_OK) return rc;
+    set_output_views(c, c->nt);
+    if (!c->side) HIPCHK(c, hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
+    c->side_busy = true;
+    HIPCHK(c, hipMemcpyAsync(c->h_nnb, c->d_nnb, (size_t)c->nt * sizeof(int),
+                             hipMemcpyDeviceToHost, c->side));
+    HIPCHK(c, hipStreamSynchronize(c->side));
+    rc = send_rows(c, c->side, kPackGroupsBeside);
+    c->rows_sent = rc == ABYSS_OK;
+    return rc;
 }
 
 // Force-kernel timing: adds up the event pairs recorded so far (waits for
@@ -583,6 +660,7 @@ void release_all(abyss_ctx_t c)
 {
     if (c->device >= 0) (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
+    if (c->side) (void)hipStreamSynchronize(c->side);
     dfree(c->d_j); hfree(c->h_j);
     dfree(c->d_tgt); dfree(c->d_out);
     c->d_list = nullptr;
@@ -603,6 +681,10 @@ void release_all(abyss_ctx_t c)
             (void)hipEventDestroy(e);
             e = nullptr;
         }
+    if (c->sums_ev) (void)hipEventDestroy(c->sums_ev);
+    c->sums_ev = nullptr;
+    if (c->side) (void)hipStreamDestroy(c->side);
+    c->side = nullptr;
     if (c->stream && c->own_stream) (void)hipStreamDestroy(c->stream);
     c->stream = nullptr;
 }
@@ -885,7 +967,8 @@ namespace abyss {
 int ctx_wait(abyss_ctx_t c)
 {
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    c->busy_tgt = c->busy_irr = c->busy_upd = false;
+    if (c->side_busy) HIPCHK(c, hipStreamSynchronize(c->side));
+    c->busy_tgt = c->busy_irr = c->busy_upd = c->side_busy = false;
     return ABYSS_OK;
 }
 
@@ -981,6 +1064,11 @@ int ctx_launch_force(abyss_ctx_t c, bool to_host)
     if (c->nt <= 0) return set_detail(c, ABYSS_ERR_INVALID_ARG, "no targets set");
     HIPCHK(c, hipSetDevice(c->device));
     c->busy_tgt = true;
+    c->rows_sent = false;
+    if (c->side_busy) {   // rows that no fetch has taken
+        int rc = ctx_wait(c);
+        if (rc != ABYSS_OK) return rc;
+    }
     if (!c->plan_valid) {
         c->plan = make_plan(c, c->nt, c->n);
         int rc = ensure_scratch(c, c->plan, c->nt);
@@ -1060,7 +1148,10 @@ int ctx_launch_force(abyss_ctx_t c, bool to_host)
     }
     c->mirror_valid = in_place || (mirrored && p.splits > 1);
     if (checked) {
-        int rc = recheck(c, p.splits > 1, mirror);
+        const bool rows_early = to_host && !c->batch_member &&
+                                c->nt > abyss::kRecheckOnDeviceMax &&
+                                row_bytes > kOneTripListBytes;
+        int rc = recheck(c, p.splits > 1, mirror, rows_early);
         if (rc != ABYSS_OK) return rc;
         c->spread_valid = true;
     }
@@ -1131,44 +1222,56 @@ namespace {
 
 // Copies the host block's acc, adot and counts and the list rows into the
 // caller's arrays; with chunks > 0 the rows of chunk k are there once
-// c->fev[k] has completed.  Large results are copied by several host
-// threads, each a slice of every chunk: one waits for the events and lets
-// the others (and itself) at the chunks that have arrived.
-hipError_t unpack_results(abyss_ctx_t c, int chunks, const int *rows, size_t stride,
-                          size_t list_bytes, double *acc, double *adot, int *nnb, int *list)
+// c->fev[k] has completed, with sums_late acc and adot, after the rows, once
+// c->sums_ev has.  Large results are copied by several host threads, each a
+// slice of every chunk: one waits for the events and lets the others (and
+// itself) at the chunks that have arrived.
+hipError_t unpack_results(abyss_ctx_t c, int chunks, bool sums_late, const int *rows,
+                          size_t stride, size_t list_bytes, double *acc, double *adot, int *nnb,
+                          int *list)
 {
     const int nt = c->nt, cap = c->cap;
     const int nchunk = std::max(chunks, 1);
+    const int steps = nchunk + (sums_late ? 1 : 0);   // the last: acc and adot
     std::atomic<int> ready{chunks > 0 ? 0 : nchunk};
-    hipError_t err = hipSuccess;   // written by part 0 before it opens the last chunk
+    hipError_t err = hipSuccess;   // written by part 0 before it opens the last step
     int parts = 1;
     const auto part = [&](int p) {
         const auto slice = [&](int a, int b, int *lo, int *hi) {
             *lo = a + (int)((long long)(b - a) * p / parts);
             *hi = a + (int)((long long)(b - a) * (p + 1) / parts);
         };
-        int lo = 0, hi = 0;
-        slice(0, nt, &lo, &hi);
-        const size_t n3 = 3 * (size_t)(hi - lo), o3 = 3 * (size_t)lo;
-        memcpy(acc + o3, c->h_res + o3, n3 * sizeof(double));
-        memcpy(adot + o3, c->h_res + 3 * (size_t)nt + o3, n3 * sizeof(double));
-        memcpy(nnb + lo, c->h_nnb + lo, (size_t)(hi - lo) * sizeof(int));
-        for (int k = 0; k < nchunk; ++k) {
-            if (p == 0 && chunks > 0) {
-                const hipError_t e = err == hipSuccess ? hipEventSynchronize(c->fev[k]) : err;
-                if (e != hipSuccess) err = e;
-                ready.store(e == hipSuccess ? k + 1 : -1, std::memory_order_release);
+        // false: a wait failed, nothing more arrives
+        const auto arrived = [&](int k) {
+            if (p == 0 && ready.load(std::memory_order_relaxed) <= k) {
+                err = hipEventSynchronize(k < nchunk ? c->fev[k] : c->sums_ev);
+                ready.store(err == hipSuccess ? k + 1 : -1, std::memory_order_release);
             }
             int r = ready.load(std::memory_order_acquire);
             while (r >= 0 && r <= k) {
                 std::this_thread::yield();
                 r = ready.load(std::memory_order_acquire);
             }
-            if (r < 0) return;   // a failed wait: nothing more arrives
+            return r >= 0;
+        };
+        const auto sums = [&]() {
+            int lo = 0, hi = 0;
+            slice(0, nt, &lo, &hi);
+            const size_t n3 = 3 * (size_t)(hi - lo), o3 = 3 * (size_t)lo;
+            memcpy(acc + o3, c->h_res + o3, n3 * sizeof(double));
+            memcpy(adot + o3, c->h_res + 3 * (size_t)nt + o3, n3 * sizeof(double));
+        };
+        int lo = 0, hi = 0;
+        slice(0, nt, &lo, &hi);
+        memcpy(nnb + lo, c->h_nnb + lo, (size_t)(hi - lo) * sizeof(int));
+        if (!sums_late) sums();
+        for (int k = 0; k < nchunk; ++k) {
+            if (!arrived(k)) return;
             slice((int)((long long)nt * k / nchunk), (int)((long long)nt * (k + 1) / nchunk), &lo,
                   &hi);
             abyss::unpack_rows(lo, hi, c->h_nnb, rows, stride, cap, list);
         }
+        if (steps > nchunk && arrived(nchunk)) sums();
     };
     if (list_bytes >= kUnpackParallelBytes) {
         parts = std::min(abyss::host_parts(), kUnpackParts);
@@ -1194,79 +1297,62 @@ int ctx_fetch_on_stream(abyss_ctx_t c, hipStream_t st, double *acc, double *adot
     // Mirrored results are in the host block already.  Other small ones:
     // acc, adot, counts and the full list rows are one contiguous block,
     // moved by one copy.  Larger ones: the counts first, then only the
-    // populated list entries, in chunks.
+    // populated list entries, in chunks; after a launch that has sent these
+    // already, acc and adot.
     const size_t full_bytes = (size_t)nt * cap * sizeof(int);
+    const size_t sums_bytes = (size_t)nt * 6 * sizeof(double);
     const bool mirrored = c->mirror_valid && st == c->stream;
+    const bool sent = c->rows_sent && st == c->stream;
     const bool one_trip = mirrored || full_bytes <= kOneTripListBytes;
-    if (!mirrored) {
-        int rc = ensure_host_rows(c, one_trip ? full_bytes : 0);
-        if (rc != ABYSS_OK) return rc;
-        set_output_views(c, nt);
-    }
-    if (!mirrored)
-        HIPCHK(c, hipMemcpyAsync(c->h_out, c->d_out,
-                                 one_trip ? packed_bytes((size_t)nt) + full_bytes
-                                          : (size_t)nt * (6 * sizeof(double) + sizeof(int)),
-                                 hipMemcpyDeviceToHost, st));
-    HIPCHK(c, hipStreamSynchronize(st));
-    if (st == c->stream) c->busy_tgt = c->busy_irr = c->busy_upd = false;
-    // populated width and overflow count, from the counts on the host
-    int width = 0, overflowed = 0;
-    size_t entries = 0;
-    for (int k = 0; k < nt; ++k) {
-        const int cnt = c->h_nnb[k];
-        const int n = std::min(cnt < 0 ? -cnt : cnt, cap);
-        overflowed += cnt < 0;
-        width = std::max(width, n);
-        entries += n;
-    }
-    const size_t list_bytes = entries * sizeof(int);
+    c->rows_sent = false;
     const int *rows = c->h_rows;
     size_t stride = cap;   // row stride of `rows`
-    int chunks = 1;        // chunks of rows still to arrive (1 when all are here)
-    if (!one_trip && width > 0) {
-        const size_t need = (size_t)nt * width * sizeof(int);
-        if (need > c->h_list_bytes) {
-            hfree(c->h_list);
-            c->h_list_bytes = 0;
-            HIPCHK(c, hipHostMalloc(&c->h_list, grow(need),
-                                    hipHostMallocMapped | hipHostMallocCoherent));
-            void *dev = nullptr;
-            HIPCHK(c, hipHostGetDevicePointer(&dev, c->h_list, 0));
-            c->h_list_dev = static_cast<int *>(dev);
-            c->h_list_bytes = grow(need);
+    if (sent) {
+        HIPCHK(c, hipMemcpyAsync(c->h_out, c->d_out, sums_bytes, hipMemcpyDeviceToHost, st));
+        if (!c->sums_ev)
+            HIPCHK(c, hipEventCreateWithFlags(&c->sums_ev, hipEventDisableTiming));
+        HIPCHK(c, hipEventRecord(c->sums_ev, st));
+    } else {
+        if (!mirrored) {
+            int rc = ensure_host_rows(c, one_trip ? full_bytes : 0);
+            if (rc != ABYSS_OK) return rc;
+            set_output_views(c, nt);
+            rows = c->h_rows;
+            HIPCHK(c, hipMemcpyAsync(c->h_out, c->d_out,
+                                     one_trip ? packed_bytes((size_t)nt) + full_bytes
+                                              : sums_bytes + (size_t)nt * sizeof(int),
+                                     hipMemcpyDeviceToHost, st));
         }
-        rows = c->h_list;
-        stride = width;
-        chunks = (int)std::min<size_t>(std::max<size_t>(1, list_bytes / kFetchChunkBytes),
-                                       std::min<size_t>(abyss_ctx_s::kFetchChunks, nt));
-        for (int k = 0; k < chunks; ++k) {
-            if (!c->fev[k])
-                HIPCHK(c, hipEventCreateWithFlags(&c->fev[k], hipEventDisableTiming));
-            const int q0 = (int)((long long)nt * k / chunks);
-            const int q1 = (int)((long long)nt * (k + 1) / chunks);
+        HIPCHK(c, hipStreamSynchronize(st));
+        if (st == c->stream) c->busy_tgt = c->busy_irr = c->busy_upd = false;
+    }
+    if (one_trip) {
+        int overflowed = 0;
+        size_t entries = 0;
+        for (int k = 0; k < nt; ++k) {
+            const int cnt = c->h_nnb[k];
+            overflowed += cnt < 0;
+            entries += std::min(cnt < 0 ? -cnt : cnt, cap);
+        }
+        c->rows_overflowed = overflowed;
+        c->rows_chunks = 0;
+        c->rows_bytes = entries * sizeof(int);
+    } else {
+        if (!sent) {
             // another stream than the context's may share the GPU with a
             // launch that fills it: the copy engine instead of a kernel
-            if (st == c->stream)
-                HIPCHK(c, abyss::launch_pack_rows(c->d_list, c->d_nnb, cap, q0, q1, c->h_list_dev,
-                                                  width, st));
-            else
-                HIPCHK(c, hipMemcpy2DAsync(c->h_list + (size_t)q0 * width,
-                                           (size_t)width * sizeof(int),
-                                           c->d_list + (size_t)q0 * cap,
-                                           (size_t)cap * sizeof(int),
-                                           (size_t)width * sizeof(int), q1 - q0,
-                                           hipMemcpyDeviceToHost, st));
-            HIPCHK(c, hipEventRecord(c->fev[k], st));
+            int rc = send_rows(c, st, st == c->stream ? INT_MAX : 0);
+            if (rc != ABYSS_OK) return rc;
         }
+        rows = c->h_list;
+        stride = c->rows_width;
     }
-    const bool arriving = rows == c->h_list && width > 0;
-    hipError_t wait = unpack_results(c, arriving ? chunks : 0, rows, stride, list_bytes, acc, adot,
-                                     nnb, list);
-    HIPCHK(c, wait);
-    if (overflowed > 0)
+    HIPCHK(c, unpack_results(c, c->rows_chunks, sent, rows, stride, c->rows_bytes, acc, adot, nnb,
+                             list));
+    if (sent) c->busy_tgt = c->busy_irr = c->busy_upd = c->side_busy = false;
+    if (c->rows_overflowed > 0)
         return set_detail(c, ABYSS_ERR_NEIGHBOR_OVERFLOW,
-                          "%d target(s) exceeded the neighbour cap %d", overflowed, cap);
+                          "%d target(s) exceeded the neighbour cap %d", c->rows_overflowed, cap);
     return ABYSS_OK;
 }
 

@@ -234,3 +234,61 @@ def test_updates_and_calls_that_do_not_wait(count):
             want = d.query(t)
             for p, q in zip(got, want):
                 assert np.array_equal(p, q)
+
+
+@pytest.mark.parametrize("tiles", [7, 8, 9])
+def test_spans_around_the_priority_rule(tiles):
+    """Four lanes per target above 32768 particles: workgroups of few tiles
+    keep equal wave priorities, from 8 tiles on they do not.  Same lists as
+    with 16 lanes per target; the FP32 runs are one tile each in both kernels,
+    so only the order of the FP64 partials differs."""
+    say(f"case: spans tiles={tiles}")
+    n, cap = 40000, 200
+    js = workloads.plummer_kroupa(n, seed=3, k_nb=80)
+    t = np.random.default_rng(tiles).permutation(n)[:300].astype(np.int32)
+    whole = (n + 255) // 256
+    out = []
+    with regf.Context(device=0, cap=cap, precision=regf.PREC_SPLIT) as c:
+        c.upload(js.m, js.x, js.v, js.r2)
+        for splits, lanes in ((-(-whole // tiles), 4), (1, 4), (1, 16)):
+            c.set_tuning(0, splits, 0, lanes)
+            out.append([a.copy() for a in c.query(t)])
+    for o in out[1:]:
+        assert np.array_equal(out[0][2], o[2]) and np.array_equal(out[0][3], o[3])
+    # 157 partials, the largest up to 1e4 times their sum
+    tol = whole * 2.0 ** -53 * 1e4
+    for p, q in zip(out[0][:2], out[1][:2]):
+        assert np.linalg.norm(p - q) <= tol * np.linalg.norm(q)
+
+
+@pytest.mark.parametrize("n,m,cap,k_nb", [
+    (20000, 4097, 256, 64),      # first block whose rows leave early
+    (20000, 20000, 256, 64),     # several chunks
+    (20000, 4097, 30, 40),       # rows small enough for one copy: not early
+    (20000, 5000, 100, 110),     # overflow
+    (9000, 4500, 1000, 5)])
+def test_rows_sent_beside_the_recomputation(n, m, cap, k_nb):
+    """A checked query of more than 4096 targets sends its list rows while the
+    flagged targets are recomputed; launch and fetch send them afterwards."""
+    say(f"case: rows early n={n} m={m} cap={cap}")
+    js = workloads.plummer_kroupa(n, seed=5, k_nb=k_nb)
+    rng = np.random.default_rng(m)
+    with regf.Context(device=0, cap=cap, precision=regf.PREC_CHECKED) as c:
+        for f in (1.0, 0.0, 1.3):   # also no neighbour at all
+            c.upload(js.m, js.x, js.v, js.r2 * f)
+            t = rng.permutation(n)[:m].astype(np.int32)
+            for _ in range(2):
+                got = [a.copy() for a in c.query(t)]
+                status, flagged = c.last_status, c.last_recheck()
+                c.set_targets(t)
+                c.launch()
+                want = c.fetch()
+                assert status == c.last_status and flagged == c.last_recheck()
+                for p, q in zip(got, want):
+                    assert np.array_equal(p, q)
+        # a launch after a query, and the list kernels behind a step
+        c.keep_lists()
+        step = c.regular_step(t, np.full(m, 1e-3), np.zeros((m, 6)))
+        for p, q in zip(step[:4], want):
+            assert np.array_equal(p, q)
+    assert flagged > 0
