@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 
+#include <type_traits>
+
 namespace abyss {
 
 // Device-resident j-set, SoA with stride `stride` (>= n).  The reference
@@ -37,6 +39,19 @@ struct FinalMirror {
     int *nnb = nullptr;      // [nt]
     int *list = nullptr;     // [nt][cap]
 };
+
+// The targets of a small block as a kernel argument (n 0: in memory).  A
+// kernel that reads them from mapped host memory waits for the link first:
+// query of 1 / 16 / 64 targets, N = 1024, 21.9 / 23.3 / 24.8 us that way,
+// 21.0 / 22.4 / 23.7 as an argument.
+constexpr int kSmallTargets = 64;
+struct SmallTargets {
+    int n;
+    int t[kSmallTargets];
+};
+struct NoSmallTargets {};
+template <int JL>
+using TargetArg = std::conditional_t<(JL >= 16), SmallTargets, NoSmallTargets>;
 
 // Checked precision's flagging done by the finalize of a split launch
 // (counter null: none): targets that need recomputation are appended to fq
@@ -192,9 +207,11 @@ hipError_t launch_batch_finalize(const ClusterDesc *cd, const int *fin_cl, const
 // kPrecRecheck (the recomputation of checked precision).
 // reset (checked precision, lanes-per-target plans): a counter the kernel
 // zeroes before any later launch on the stream reads it.
+// small: host copy of tgt for a launch that is not captured (null: none); 16
+// and 64 lanes per target take up to kSmallTargets of it as an argument.
 hipError_t launch_regf(const JState &js, const int *tgt, int nt, const Plan &plan,
                        const QueryOut &out, int cap, int prec, hipStream_t st,
-                       int *reset = nullptr);
+                       int *reset = nullptr, const int *small = nullptr);
 
 // Internal mode of launch_regf: the neighbour test of split precision (FP32
 // r^2 of the rounded differences, so the regular set is the same) with FP64

@@ -32,6 +32,7 @@
 #include "regf_internal.h"
 
 #include <limits.h>
+#include <string.h>
 
 namespace abyss {
 namespace {
@@ -782,6 +783,21 @@ __device__ __forceinline__ void regf_body_jl(const JState &js, const int *__rest
     const int j1 = min(js.n, j0 + jspan);
     const int q = bx * (WPB * TW) + (tid >> 6) * TW + g;
     const bool loader = TILE == 64 * WPB || tid < TILE;
+    const int ntile = (j1 - j0 + TILE - 1) / TILE;
+
+    // The first tile is asked for before the targets, whose list may be in
+    // host memory and whose particles are a second load after it: query of one
+    // target, N = 1024, 22.4 -> 21.9 us; force kernel, N = 65536, 1000 targets
+    // 80.7 -> 78.8 us, King N = 262144, every target, 51.04 -> 50.88 ms.
+    TileLoader<MT> ld;
+    TileLoader<MT> lr[ONE_SHOT ? R : 1];
+    if constexpr (ONE_SHOT) {
+        // every load in flight before the first store (ntile <= 1)
+#pragma unroll
+        for (int r = 0; r < R; ++r) lr[r].load(js, j0 + r * 64 * WPB + tid, j1);
+    } else if (ntile > 0 && loader) {
+        ld.load(js, j0 + tid, j1);
+    }
 
     JLLane L;
     L.sub = lane % JL;
@@ -818,20 +834,13 @@ __device__ __forceinline__ void regf_body_jl(const JState &js, const int *__rest
         }
     };
 
-    const int ntile = (j1 - j0 + TILE - 1) / TILE;
     // a wave without targets loads its share of every tile and meets every
     // barrier, but evaluates nothing
     const bool wave_busy = __any(q < nt);
-    TileLoader<MT> ld;
     if constexpr (ONE_SHOT) {
-        // every load in flight before the first store (ntile <= 1)
-        TileLoader<MT> lr[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) lr[r].load(js, j0 + r * 64 * WPB + tid, j1);
 #pragma unroll
         for (int r = 0; r < R; ++r) lr[r].store(s_pos[0], s_m[0], r * 64 * WPB + tid);
     } else if (ntile > 0 && loader) {
-        ld.load(js, j0 + tid, j1);
         ld.store(s_pos[0], s_m[0], tid);
     }
     __syncthreads();
@@ -941,12 +950,15 @@ __device__ __forceinline__ void xcd_place(int id, int total, int gx, int &bx, in
 // A one-shot tile's 52 KB of LDS (56 KB with FP64 masses) holds 3 (2)
 // workgroups per CU, so it asks for 3 (2).
 // Grid: gx * splits workgroups on x (xcd_place).
+// small (16 and 64 lanes per target): the targets of a small block, instead of
+// tgt (SmallTargets).
 template <int JL, int TM, bool EST, int TILE = kTile, int WPB = 4, bool MASKED = false,
           bool PRIO = JL == 16>
 __global__ __launch_bounds__(64 * WPB)
 __attribute__((amdgpu_waves_per_eu(TILE > 64 * WPB ? (TM == 0 ? 3 : 2) : 5, 8)))
 void regf_kernel_jl(JState js, const int *__restrict__ tgt, int nt, int jspan, QueryOut out,
-                    int cap, int final_counts, int *__restrict__ reset, int gx, int splits)
+                    int cap, int final_counts, int *__restrict__ reset, int gx, int splits,
+                    TargetArg<JL> small)
 {
     if (reset && blockIdx.x == 0 && threadIdx.x == 0) *reset = 0;
     // a one-shot tile (TILE > 64 WPB) has a single buffer
@@ -955,6 +967,7 @@ void regf_kernel_jl(JState js, const int *__restrict__ tgt, int nt, int jspan, Q
     __shared__ typename TermMass<TM>::type s_m[NB][TILE];
     int bx, s;
     xcd_place(blockIdx.x, gx * splits, gx, bx, s);
+    if constexpr (JL >= 16) tgt = small.n > 0 ? small.t : tgt;
     regf_body_jl<JL, TM, EST, TILE, WPB, MASKED, PRIO>(js, tgt, nt, jspan, out, cap, final_counts,
                                                        bx, s, 0, nt, s_pos, s_m);
 }
@@ -1537,48 +1550,66 @@ hipError_t launch_t(const JState &js, const int *tgt, int nt, const Plan &p, con
     return hipGetLastError();
 }
 
+// The kernel's copy of a small block's targets (small: on the host, or null).
+template <int JL>
+TargetArg<JL> target_arg(const int *small, int nt)
+{
+    TargetArg<JL> a{};
+    if constexpr (JL >= 16) {
+        if (small && nt <= kSmallTargets) {
+            a.n = nt;
+            memcpy(a.t, small, (size_t)nt * sizeof(int));
+        }
+    }
+    return a;
+}
+
 // Term mode 0 with the plan's shape (j-tile, wave64s per workgroup).
 template <int JL, bool EST, int TILE, int WPB>
 void launch_shape(const JState &js, const int *tgt, int nt, const Plan &p, const QueryOut &out,
-                  int cap, int fc, int *reset, hipStream_t st)
+                  int cap, int fc, int *reset, const int *small,
+          hipStream_t st)
 {
     if constexpr (JL == 4) {
         if (js.n <= kMaskedMax) {
             hipLaunchKernelGGL((regf_kernel_jl<JL, 0, EST, TILE, WPB, true>),
                                dim3(p.grid_x * p.splits), dim3(64 * WPB), 0, st, js, tgt, nt,
-                               p.jspan, out, cap, fc, reset, p.grid_x, p.splits);
+                               p.jspan, out, cap, fc, reset, p.grid_x, p.splits,
+                               target_arg<JL>(small, nt));
             return;
         }
         if constexpr (TILE == kTile && WPB == 4) {
             if (p.jspan >= kPrioSpan) {
                 hipLaunchKernelGGL((regf_kernel_jl<JL, 0, EST, TILE, WPB, false, true>),
                                    dim3(p.grid_x * p.splits), dim3(64 * WPB), 0, st, js, tgt, nt,
-                                   p.jspan, out, cap, fc, reset, p.grid_x, p.splits);
+                                   p.jspan, out, cap, fc, reset, p.grid_x, p.splits,
+                               target_arg<JL>(small, nt));
                 return;
             }
         }
     }
     hipLaunchKernelGGL((regf_kernel_jl<JL, 0, EST, TILE, WPB>), dim3(p.grid_x * p.splits),
                        dim3(64 * WPB), 0, st, js, tgt, nt, p.jspan, out, cap, fc, reset, p.grid_x,
-                       p.splits);
+                       p.splits, target_arg<JL>(small, nt));
 }
 
 template <int JL, bool EST>
 hipError_t launch_mode0(const JState &js, const int *tgt, int nt, const Plan &p,
-                        const QueryOut &out, int cap, int fc, int *reset, hipStream_t st)
+                        const QueryOut &out, int cap, int fc, int *reset, const int *small,
+          hipStream_t st)
 {
     switch (p.tile * 8 + p.wpb) {
-        case 256 * 8 + 4: launch_shape<JL, EST, 256, 4>(js, tgt, nt, p, out, cap, fc, reset, st); break;
-        case 128 * 8 + 4: launch_shape<JL, EST, 128, 4>(js, tgt, nt, p, out, cap, fc, reset, st); break;
-        case 64 * 8 + 4: launch_shape<JL, EST, 64, 4>(js, tgt, nt, p, out, cap, fc, reset, st); break;
-        case 128 * 8 + 2: launch_shape<JL, EST, 128, 2>(js, tgt, nt, p, out, cap, fc, reset, st); break;
-        case 64 * 8 + 2: launch_shape<JL, EST, 64, 2>(js, tgt, nt, p, out, cap, fc, reset, st); break;
-        case 64 * 8 + 1: launch_shape<JL, EST, 64, 1>(js, tgt, nt, p, out, cap, fc, reset, st); break;
+        case 256 * 8 + 4: launch_shape<JL, EST, 256, 4>(js, tgt, nt, p, out, cap, fc, reset, small, st); break;
+        case 128 * 8 + 4: launch_shape<JL, EST, 128, 4>(js, tgt, nt, p, out, cap, fc, reset, small, st); break;
+        case 64 * 8 + 4: launch_shape<JL, EST, 64, 4>(js, tgt, nt, p, out, cap, fc, reset, small, st); break;
+        case 128 * 8 + 2: launch_shape<JL, EST, 128, 2>(js, tgt, nt, p, out, cap, fc, reset, small, st); break;
+        case 64 * 8 + 2: launch_shape<JL, EST, 64, 2>(js, tgt, nt, p, out, cap, fc, reset, small, st); break;
+        case 64 * 8 + 1: launch_shape<JL, EST, 64, 1>(js, tgt, nt, p, out, cap, fc, reset, small, st); break;
         case 1024 * 8 + 4:
             // one-shot tiles: every split within one tile (fold at 16 or 64 steps)
             if constexpr (JL >= 16) {
                 if (p.jspan > 1024) return hipErrorInvalidValue;
-                launch_shape<JL, EST, 1024, 4>(js, tgt, nt, p, out, cap, fc, reset, st);
+                launch_shape<JL, EST, 1024, 4>(js, tgt, nt, p, out, cap, fc, reset, small, st);
                 break;
             }
             return hipErrorInvalidValue;
@@ -1590,7 +1621,8 @@ hipError_t launch_mode0(const JState &js, const int *tgt, int nt, const Plan &p,
 // tm: term mode; est: the spread estimate of checked precision (mode 0)
 template <int JL>
 hipError_t launch_jl(const JState &js, const int *tgt, int nt, const Plan &p, const QueryOut &out,
-                     int cap, int tm, bool est, int *reset, hipStream_t st)
+                     int cap, int tm, bool est, int *reset, const int *small,
+          hipStream_t st)
 {
     // one workgroup per (target block, split) on a 1-D grid (xcd_place)
     if ((long long)p.grid_x * p.splits > 0x7fffffffLL) return hipErrorInvalidValue;
@@ -1602,25 +1634,28 @@ hipError_t launch_jl(const JState &js, const int *tgt, int nt, const Plan &p, co
             if (p.jspan > kTileOneShot) return hipErrorInvalidValue;
             hipLaunchKernelGGL((regf_kernel_jl<JL, 3, false, kTileOneShot, 4>), grid,
                                dim3(kBlock), 0, st, js, tgt, nt, p.jspan, out, cap, fc, reset,
-                               p.grid_x, p.splits);
+                               p.grid_x, p.splits, target_arg<JL>(small, nt));
             return hipGetLastError();
         }
         return hipErrorInvalidValue;
     }
     if (tm != 0 && (p.tile != kTile || p.wpb != 4)) return hipErrorInvalidValue;
     if (tm == 0 && est)
-        return launch_mode0<JL, true>(js, tgt, nt, p, out, cap, fc, reset, st);
+        return launch_mode0<JL, true>(js, tgt, nt, p, out, cap, fc, reset, small, st);
     else if (tm == 0)
-        return launch_mode0<JL, false>(js, tgt, nt, p, out, cap, fc, reset, st);
+        return launch_mode0<JL, false>(js, tgt, nt, p, out, cap, fc, reset, small, st);
     else if (tm == 1)
         hipLaunchKernelGGL((regf_kernel_jl<JL, 1, false, kTile, 4, JL == 4>), grid, dim3(kBlock), 0, st, js, tgt,
-                           nt, p.jspan, out, cap, fc, reset, p.grid_x, p.splits);
+                           nt, p.jspan, out, cap, fc, reset, p.grid_x, p.splits,
+                               target_arg<JL>(small, nt));
     else if (tm == 2)
         hipLaunchKernelGGL((regf_kernel_jl<JL, 2, false, kTile, 4, JL == 4>), grid, dim3(kBlock), 0, st, js, tgt,
-                           nt, p.jspan, out, cap, fc, reset, p.grid_x, p.splits);
+                           nt, p.jspan, out, cap, fc, reset, p.grid_x, p.splits,
+                               target_arg<JL>(small, nt));
     else
         hipLaunchKernelGGL((regf_kernel_jl<JL, 3, false, kTile, 4, JL == 4>), grid, dim3(kBlock), 0, st, js, tgt,
-                           nt, p.jspan, out, cap, fc, reset, p.grid_x, p.splits);
+                           nt, p.jspan, out, cap, fc, reset, p.grid_x, p.splits,
+                               target_arg<JL>(small, nt));
     return hipGetLastError();
 }
 
@@ -1660,16 +1695,17 @@ bool shape_supported(int tile, int wpb)
 }
 
 hipError_t launch_regf(const JState &js, const int *tgt, int nt, const Plan &p,
-                       const QueryOut &out, int cap, int prec, hipStream_t st, int *reset)
+                       const QueryOut &out, int cap, int prec, hipStream_t st, int *reset,
+                       const int *small)
 {
     if (!variant_supported(prec, p.ipl, p.unroll, p.jl)) return hipErrorInvalidValue;
     const int tm = term_mode(prec);
     const bool est = prec == ABYSS_PREC_CHECKED;
     if (est && !out.spread) return hipErrorInvalidValue;
     if (p.jl > 1 && !shape_supported(p.tile, p.wpb)) return hipErrorInvalidValue;
-    if (p.jl == 4) return launch_jl<4>(js, tgt, nt, p, out, cap, tm, est, reset, st);
-    if (p.jl == 16) return launch_jl<16>(js, tgt, nt, p, out, cap, tm, est, reset, st);
-    if (p.jl == 64) return launch_jl<64>(js, tgt, nt, p, out, cap, tm, est, reset, st);
+    if (p.jl == 4) return launch_jl<4>(js, tgt, nt, p, out, cap, tm, est, reset, small, st);
+    if (p.jl == 16) return launch_jl<16>(js, tgt, nt, p, out, cap, tm, est, reset, small, st);
+    if (p.jl == 64) return launch_jl<64>(js, tgt, nt, p, out, cap, tm, est, reset, small, st);
     if (reset || p.tile != kTile || p.wpb != 4)
         return hipErrorInvalidValue;   // the lanes-per-target kernels only
     if (prec == ABYSS_PREC_FP64) {

@@ -1128,7 +1128,8 @@ int ctx_launch_force(abyss_ctx_t c, bool to_host)
     // own)
     HIPCHK(c, abyss::launch_regf(c->js, c->tgt, c->nt, p, p.splits == 1 ? fin : part, c->cap,
                                  direct ? abyss::kPrecRecheck : c->precision, c->stream,
-                                 checked ? c->chk_counters : nullptr));
+                                 checked ? c->chk_counters : nullptr,
+                                 to_host && c->tgt == c->h_tgt_dev ? c->h_tgt : nullptr));
     if (c->ktiming) {
         HIPCHK(c, hipEventRecord(c->kev[2 * c->kev_used + 1], c->stream));
         c->kev_used += 1;

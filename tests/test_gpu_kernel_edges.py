@@ -292,3 +292,26 @@ def test_rows_sent_beside_the_recomputation(n, m, cap, k_nb):
         for p, q in zip(step[:4], want):
             assert np.array_equal(p, q)
     assert flagged > 0
+
+
+@pytest.mark.parametrize("prec", [regf.PREC_SPLIT, regf.PREC_CHECKED, regf.PREC_REFINED])
+@pytest.mark.parametrize("n,lanes", [(1024, 0), (3000, 16), (9000, 64)])
+def test_small_blocks_as_arguments(n, lanes, prec):
+    """A query of up to 64 targets passes them to the kernel, a launch leaves
+    them in memory, where a later block of the same size is found."""
+    say(f"case: small blocks n={n} lanes={lanes} precision={prec}")
+    js = workloads.plummer_kroupa(n, seed=2, k_nb=20)
+    rng = np.random.default_rng(n)
+    with regf.Context(device=0, cap=64, precision=prec) as c:
+        c.upload(js.m, js.x, js.v, js.r2)
+        c.set_tuning(0, 0, 0, lanes)
+        for nt in (1, 63, 64, 65, 64, 2, 3):
+            t = rng.permutation(n)[:nt].astype(np.int32)
+            got = [a.copy() for a in c.query(t)]
+            c.set_targets(t)
+            c.launch()
+            want = c.fetch()
+            again = c.query(t)
+            for p, q, r in zip(got, want, again):
+                assert np.array_equal(p, q) and np.array_equal(p, r)
+            assert (got[2] != 0).any()
