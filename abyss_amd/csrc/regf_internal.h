@@ -84,6 +84,7 @@ struct Plan {
     // checked precision of a small block: every target in FP64 terms in one
     // pass (kPrecRecheck arithmetic, with lists), no flag or recomputation
     bool fp64_terms = false;
+    bool merged = false;   // one split whose results go through the merge all the same
 };
 // Checked-precision blocks of at most this many targets (outside batches)
 // run in FP64 terms in one pass: below ~1000 targets that is faster than

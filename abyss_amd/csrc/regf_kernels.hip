@@ -1546,7 +1546,7 @@ hipError_t launch_t(const JState &js, const int *tgt, int nt, const Plan &p, con
 {
     dim3 grid(p.grid_x, p.splits);
     hipLaunchKernelGGL((regf_kernel<IPL, U, F64>), grid, dim3(kBlock), 0, st, js, tgt, nt,
-                       p.jspan, out, cap, p.splits == 1 ? 1 : 0);
+                       p.jspan, out, cap, p.splits == 1 && !p.merged ? 1 : 0);
     return hipGetLastError();
 }
 
@@ -1627,7 +1627,7 @@ hipError_t launch_jl(const JState &js, const int *tgt, int nt, const Plan &p, co
     // one workgroup per (target block, split) on a 1-D grid (xcd_place)
     if ((long long)p.grid_x * p.splits > 0x7fffffffLL) return hipErrorInvalidValue;
     dim3 grid(p.grid_x * p.splits);
-    const int fc = p.splits == 1 ? 1 : 0;
+    const int fc = p.splits == 1 && !p.merged ? 1 : 0;
     if (tm == 3 && p.tile == kTileOneShot && p.wpb == 4) {
         // a checked block in FP64 terms in one pass, every split one tile
         if constexpr (JL >= 16) {

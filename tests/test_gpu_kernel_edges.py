@@ -315,3 +315,33 @@ def test_small_blocks_as_arguments(n, lanes, prec):
             for p, q, r in zip(got, want, again):
                 assert np.array_equal(p, q) and np.array_equal(p, r)
             assert (got[2] != 0).any()
+
+
+@pytest.mark.parametrize("prec", [regf.PREC_SPLIT, regf.PREC_CHECKED, regf.PREC_MIXED,
+                                  regf.PREC_REFINED, regf.PREC_FP64])
+@pytest.mark.parametrize("n,m,cap,k_nb", [(67, 65, 64, 20), (300, 300, 64, 20),
+                                          (1024, 257, 30, 40), (1900, 1900, 256, 40)])
+def test_one_split_through_the_merge(n, m, cap, k_nb, prec):
+    """A query of one split and more than 64 targets merges it into host
+    memory, a launch leaves it where the kernel wrote it: the same bytes, and
+    the same behind a step of resident lists."""
+    say(f"case: one split n={n} m={m} precision={prec}")
+    js = workloads.plummer_kroupa(n, seed=9, k_nb=k_nb)
+    t = np.random.default_rng(m).permutation(n)[:m].astype(np.int32)
+    with regf.Context(device=0, cap=cap, precision=prec) as c:
+        c.upload(js.m, js.x, js.v, js.r2)
+        c.set_tuning(0, 1, 0, 0)
+        got = [a.copy() for a in c.query(t)]
+        status, flagged = c.last_status, c.last_recheck()
+        assert c.plan()["j_splits"] == 1
+        c.set_targets(t)
+        c.launch()
+        want = c.fetch()
+        assert status == c.last_status and flagged == c.last_recheck()
+        c.keep_lists()
+        step = c.regular_step(t, np.full(m, 1e-3), np.zeros((m, 6)))
+        acc, adot = c.irregular(t)
+    for p, q, r in zip(got, want, step):
+        assert np.array_equal(p, q) and np.array_equal(p, r)
+    assert np.array_equal(step[4][:, 12:15], acc) and np.array_equal(step[4][:, 15:], adot)
+    assert (got[2] < 0).any() == (cap < k_nb)
