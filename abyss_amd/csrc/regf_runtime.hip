@@ -1096,14 +1096,16 @@ int ctx_launch_force(abyss_ctx_t c, bool to_host)
     // every entry of the rows, or two copies with a host wait between them.
     // Query, targets of N: 300 of 300 49.5 -> 41 us, 256 of 1024 41 -> 33.8,
     // 1000 of 1024 75 -> 57 (split precision 63.5 -> 47.5), 2000 of 2000 100
-    // -> 79.
+    // -> 79.  Not beyond the limit of the split scratch.
     const size_t row_bytes = (size_t)c->nt * c->cap * sizeof(int);
     const bool small = c->nt <= kMappedTargets && row_bytes <= kOneTripListBytes;
-    const bool mirrored = !c->batch_member &&
-                          (small || (to_host && c->nt <= kQueryMirrorTargets &&
-                                     row_bytes <= kQueryMirrorRowBytes));
-    p.merged = mirrored && !small && p.splits == 1;
+    const bool fits = !c->batch_member &&
+                      (small || (to_host && c->nt <= kQueryMirrorTargets &&
+                                 row_bytes <= kQueryMirrorRowBytes));
+    p.merged = fits && !small && p.splits == 1 &&
+               row_bytes + (size_t)c->nt * (6 * sizeof(double) + sizeof(int)) <= c->scratch_limit;
     const bool merge = p.splits > 1 || p.merged;
+    const bool mirrored = fits && (small || merge);
     if (mirrored) {
         int rc = ensure_host_rows(c, row_bytes);
         if (rc != ABYSS_OK) return rc;

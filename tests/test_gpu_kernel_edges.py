@@ -345,3 +345,23 @@ def test_one_split_through_the_merge(n, m, cap, k_nb, prec):
         assert np.array_equal(p, q) and np.array_equal(p, r)
     assert np.array_equal(step[4][:, 12:15], acc) and np.array_equal(step[4][:, 15:], adot)
     assert (got[2] < 0).any() == (cap < k_nb)
+
+
+@pytest.mark.parametrize("prec", [regf.PREC_SPLIT, regf.PREC_CHECKED])
+def test_one_split_at_the_scratch_limit(prec):
+    """A query whose one split does not fit the scratch limit leaves it where
+    the kernel wrote it: the same bytes."""
+    say(f"case: scratch limit precision={prec}")
+    n, m = 1000, 700
+    js = workloads.plummer_kroupa(n, seed=9, k_nb=40)
+    t = np.random.default_rng(1).permutation(n)[:m].astype(np.int32)
+    out = []
+    for limit in (2 << 30, 1):
+        with regf.Context(device=0, cap=100, precision=prec) as c:
+            c.set_scratch_limit(limit)
+            c.upload(js.m, js.x, js.v, js.r2)
+            c.set_tuning(0, 1, 0, 16)
+            out.append([a.copy() for a in c.query(t)])
+            assert c.plan()["j_splits"] == 1
+    for p, q in zip(*out):
+        assert np.array_equal(p, q)
