@@ -1016,6 +1016,7 @@ int ctx_set_targets(abyss_ctx_t c, int nt, const int *targets, TargetWait wait)
     c->nt = nt;
     c->counts_valid = false;   // counts belong to the next launch
     c->mirror_valid = false;
+    c->rows_sent = false;
     c->spread_valid = false;
     c->plan = make_plan(c, nt, c->n);
     rc = ensure_scratch(c, c->plan, nt);
