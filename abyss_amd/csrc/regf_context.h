@@ -37,6 +37,10 @@ struct abyss_ctx_s {
     // no caller can put work of its own on the stream (the drop-in calls'
     // context), so the flags tell all there is
     bool closed = false;
+    // A caller's capture has recorded work of this context, which it may
+    // replay at any time between calls: calls then keep to the buffers and the
+    // waits that such work can rely on (ctx_launch_force, ctx_set_targets).
+    bool captured = false;
     int *d_tgt = nullptr, *h_tgt = nullptr;
     // h_tgt is mapped, coherent pinned memory; h_tgt_dev is its device
     // address.  `tgt` is the target array the kernels read: h_tgt_dev for
@@ -172,7 +176,7 @@ int ctx_fetch_on_stream(abyss_ctx_t c, hipStream_t st, double *acc, double *adot
 unsigned long long ctx_device_bytes(abyss_ctx_t c);
 // abyss_ctx_launch without keeping the resident lists (force kernels only).
 // to_host: a fetch follows, so blocks of up to kQueryMirrorTargets targets
-// also write their results to mapped host memory.
+// also write their results to mapped host memory, small ones only there.
 int ctx_launch_force(abyss_ctx_t c, bool to_host = false);
 // After a launch: copies its neighbour rows into the resident per-particle
 // lists when they are enabled (no-op otherwise).
@@ -187,4 +191,6 @@ enum class TargetWait { kStream, kUse, kNone };
 int ctx_set_targets(abyss_ctx_t c, int nt, const int *targets, TargetWait wait);
 // Waits for the context's stream.
 int ctx_wait(abyss_ctx_t c);
+// Whether a caller's capture is recording the context's stream.
+int ctx_capturing(abyss_ctx_t c, bool *capturing);
 }  // namespace abyss

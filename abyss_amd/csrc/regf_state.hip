@@ -200,13 +200,13 @@ int abyss_ctx_update_state(abyss_ctx_t c, int count, const int *idx, const doubl
     }
     if (hipSetDevice(c->device) != hipSuccess) return ABYSS_ERR_HIP;
     // a captured update would read whatever the staging holds at its replays
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(c->stream, &capture) != hipSuccess ||
-        capture != hipStreamCaptureStatusNone)
-        return ABYSS_ERR_HIP;
+    bool capturing = false;
+    int rc = abyss::ctx_capturing(c, &capturing);
+    if (rc != ABYSS_OK) return rc;
+    if (capturing) return ABYSS_ERR_HIP;
     // staging from a previous update may still be in flight
     if (c->busy_upd) {
-        int rc = abyss::ctx_wait(c);
+        rc = abyss::ctx_wait(c);
         if (rc != ABYSS_OK) return rc;
     }
     const size_t rec_bytes = (size_t)count * kStateDoubles * sizeof(double);

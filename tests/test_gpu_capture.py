@@ -1,0 +1,89 @@
+"""Launches recorded into a HIP graph by the caller (abyss_ctx_stream) and
+replayed between other calls on the context: every replay leaves what an
+eager launch of the same targets on the same j-set leaves."""
+import ctypes
+import sys
+
+import numpy as np
+import pytest
+
+from abyss_amd import regf, workloads
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*a):
+    print(*a, flush=True)
+    sys.stdout.flush()
+
+
+class Graph:
+    """What a `with` block enqueues on a context's stream, as a graph."""
+
+    def __init__(self, ctx):
+        self.lib = ctypes.CDLL("libamdhip64.so")
+        self.stream = ctypes.c_void_p(ctx.stream)
+        self.graph, self.exec = ctypes.c_void_p(), ctypes.c_void_p()
+
+    def __enter__(self):
+        # the default mode: calls that may wait or allocate are refused
+        assert self.lib.hipStreamBeginCapture(self.stream, 0) == 0
+        return self
+
+    def __exit__(self, kind, *a):
+        rc = self.lib.hipStreamEndCapture(self.stream, ctypes.byref(self.graph))
+        if kind is None:
+            assert rc == 0
+            assert self.lib.hipGraphInstantiate(ctypes.byref(self.exec), self.graph, None, None,
+                                                ctypes.c_size_t(0)) == 0
+
+    def replay(self):
+        assert self.lib.hipGraphLaunch(self.exec, self.stream) == 0
+
+    def free(self):
+        self.lib.hipStreamSynchronize(self.stream)
+        if self.exec:
+            self.lib.hipGraphExecDestroy(self.exec)
+        if self.graph:
+            self.lib.hipGraphDestroy(self.graph)
+
+
+def same(a, b):
+    return all(np.array_equal(p, q) for p, q in zip(a, b))
+
+
+@pytest.mark.parametrize("prec", [regf.PREC_SPLIT, regf.PREC_CHECKED])
+@pytest.mark.parametrize("n,nt", [(1024, 1), (1024, 64), (20000, 16), (20000, 300)])
+def test_replays_between_other_calls(n, nt, prec):
+    """One split and several, lists of up to 64 targets and longer ones."""
+    if prec == regf.PREC_CHECKED and nt > 256:
+        pytest.skip("allocates the checked pass's buffers inside the launch")
+    say(f"case: replay n={n} targets={nt} precision={prec}")
+    js = [workloads.plummer_kroupa(n, seed=s, k_nb=30) for s in (1, 2)]
+    rng = np.random.default_rng(n + nt)
+    pick = [rng.permutation(n)[:nt].astype(np.int32) for _ in range(4)]
+    with regf.Context(device=0, cap=64, precision=prec) as c, \
+            regf.Context(device=0, cap=64, precision=prec) as d:
+        want = {}
+        for k, s in enumerate(js):
+            d.upload(s.m, s.x, s.v, s.r2)
+            for i, t in enumerate(pick):
+                want[k, i] = [a.copy() for a in d.query(t)]
+        c.upload(js[0].m, js[0].x, js[0].v, js[0].r2)
+        c.set_targets(pick[0])
+        c.launch()
+        assert same(c.fetch(), want[0, 0])
+        g = Graph(c)
+        with g:
+            c.launch()
+        for i in (1, 2, 3):
+            c.set_targets(pick[i])
+            g.replay()
+            assert same(c.fetch(), want[0, i])
+            # a query of the same targets, then a replay on another j-set
+            assert same(c.query(pick[i]), want[0, i])
+            c.upload(js[1].m, js[1].x, js[1].v, js[1].r2)
+            g.replay()
+            assert same(c.fetch(), want[1, i])
+            c.upload(js[0].m, js[0].x, js[0].v, js[0].r2)
+        g.free()
