@@ -49,7 +49,8 @@ struct abyss_ctx_s {
     // per-target results (device block and pinned host mirror, same
     // layout): acc [nt][3] | adot [nt][3] | nnb [nt] | pad to 256 B | list
     // rows [nt][cap]; the pointers below are views of d_out / h_out for the
-    // current nt (the host mirror holds rows only up to the one-copy size)
+    // current nt (the host mirror holds the rows that fit one copy, or those
+    // that a query's last kernels write there)
     char *d_out = nullptr, *h_out = nullptr;
     size_t h_row_bytes = 0;   // list rows h_out has room for
     double *d_acc = nullptr, *d_adot = nullptr;

@@ -142,8 +142,6 @@ void set_output_views(abyss_ctx_t c, int nt)
     c->d_adot = c->d_acc + 3 * n;
     c->d_nnb = reinterpret_cast<int *>(c->d_adot + 3 * n);
     c->d_list = reinterpret_cast<int *>(c->d_out + packed_bytes(n));
-    c->mirror = abyss::FinalMirror{};
-    if (!c->h_out) return;
     c->h_res = reinterpret_cast<double *>(c->h_out);
     c->h_nnb = reinterpret_cast<int *>(c->h_res + 6 * n);
     c->h_rows = reinterpret_cast<int *>(c->h_out + packed_bytes(n));
@@ -155,10 +153,13 @@ void set_output_views(abyss_ctx_t c, int nt)
 }
 
 // The mapped host block of t_capacity targets' packed results with room for
-// at least `bytes` of list rows (no launch that writes it may be in flight).
+// at least `bytes` of list rows (no launch that writes it may be in flight,
+// nor one that a caller may replay: those ask for no more than the first
+// size).  Only with the targets: a launch that a caller records may not
+// allocate.
 int ensure_host_rows(abyss_ctx_t c, size_t bytes)
 {
-    if (c->h_out && bytes <= c->h_row_bytes) return ABYSS_OK;
+    if (c->h_out_dev && bytes <= c->h_row_bytes) return ABYSS_OK;
     hfree(c->h_out);
     c->h_out_dev = nullptr;
     c->h_row_bytes = 0;
@@ -178,7 +179,8 @@ int ensure_host_rows(abyss_ctx_t c, size_t bytes)
     return ABYSS_OK;
 }
 
-int ensure_outputs(abyss_ctx_t c, int nt)
+// row_bytes: list rows that the coming launch writes to the host block.
+int ensure_outputs(abyss_ctx_t c, int nt, size_t row_bytes)
 {
     if ((size_t)nt > c->t_capacity) {
         size_t cap_t = grow((size_t)nt);
@@ -201,15 +203,18 @@ int ensure_outputs(abyss_ctx_t c, int nt)
         c->h_tgt_dev = static_cast<const int *>(dev);
         c->t_capacity = cap_t;
     }
-    // a batch member's results may be fetched while other launches run, so
-    // its host block is allocated here; a context's by the launch or the
-    // fetch that uses it, at the size that takes
-    if (c->batch_member) {
-        int rc = ensure_host_rows(c, 0);
-        if (rc != ABYSS_OK) return rc;
-    }
+    int rc = ensure_host_rows(c, row_bytes);
+    if (rc != ABYSS_OK) return rc;
     set_output_views(c, nt);
     return ABYSS_OK;
+}
+
+// List rows of a query that its last kernels write to the host block (0: the
+// fetch moves them).
+size_t query_mirror_rows(abyss_ctx_t c, int nt)
+{
+    const size_t bytes = (size_t)nt * c->cap * sizeof(int);
+    return nt <= kQueryMirrorTargets && bytes <= kQueryMirrorRowBytes ? bytes : 0;
 }
 
 // Plan for nt targets against n j under precision `prec`; list rows of
@@ -628,9 +633,6 @@ int recheck(abyss_ctx_t c, bool flagged, const abyss::FinalMirror &mirror, bool 
     int rc = recompute_flagged(c, c->h_chk[0], mirror);
     if (rc != ABYSS_OK || !rows_early) return rc;
     // the merge has finished, so the side stream need not wait for it
-    rc = ensure_host_rows(c, 0);
-    if (rc != ABYSS_OK) return rc;
-    set_output_views(c, c->nt);
     if (!c->side) HIPCHK(c, hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
     c->side_busy = true;
     HIPCHK(c, hipMemcpyAsync(c->h_nnb, c->d_nnb, (size_t)c->nt * sizeof(int),
@@ -1004,8 +1006,15 @@ int ctx_set_targets(abyss_ctx_t c, int nt, const int *targets, TargetWait wait)
         (wait == TargetWait::kUse &&
          (c->busy_tgt || (size_t)nt > c->t_capacity || (!c->closed && c->tgt == c->h_tgt_dev))))
         rc = ctx_wait(c);
-    if (rc == ABYSS_OK) rc = ensure_outputs(c, nt);
+    // a query's results may go to the host block; that stays where it is once
+    // a recorded launch may write it
+    const size_t rows = wait == TargetWait::kUse && !c->captured ? query_mirror_rows(c, nt) : 0;
     if (rc != ABYSS_OK) return rc;
+    rc = ensure_outputs(c, nt, rows);
+    if (rc != ABYSS_OK) {
+        c->nt = 0;   // the last targets' buffers may be gone
+        return rc;
+    }
     memcpy(c->h_tgt, targets, (size_t)nt * sizeof(int));
     c->busy_tgt = true;   // until the stream is next waited for
     if (nt <= kMappedTargets || c->batch_member) {
@@ -1120,17 +1129,12 @@ int ctx_launch_force(abyss_ctx_t c, bool to_host)
     const size_t row_bytes = (size_t)c->nt * c->cap * sizeof(int);
     const bool small = c->nt <= kMappedTargets && row_bytes <= kOneTripListBytes;
     const bool fits = !c->batch_member &&
-                      (small || (to_host && c->nt <= kQueryMirrorTargets &&
-                                 row_bytes <= kQueryMirrorRowBytes));
+                      (small || (to_host && query_mirror_rows(c, c->nt) > 0));
     p.merged = fits && !small && p.splits == 1 &&
                row_bytes + (size_t)c->nt * (6 * sizeof(double) + sizeof(int)) <= c->scratch_limit;
     const bool merge = p.splits > 1 || p.merged;
     const bool in_place = to_host && fits && small && !merge && !checked;
     const bool mirrored = in_place || (fits && merge);
-    if (mirrored) {
-        int rc = ensure_host_rows(c, row_bytes);
-        if (rc != ABYSS_OK) return rc;
-    }
     if (p.merged) {
         int rc = ensure_scratch(c, p, c->nt);
         if (rc != ABYSS_OK) return rc;
@@ -1349,10 +1353,7 @@ int ctx_fetch_on_stream(abyss_ctx_t c, hipStream_t st, double *acc, double *adot
         HIPCHK(c, hipEventRecord(c->sums_ev, st));
     } else {
         if (!mirrored) {
-            int rc = ensure_host_rows(c, one_trip ? full_bytes : 0);
-            if (rc != ABYSS_OK) return rc;
             set_output_views(c, nt);
-            rows = c->h_rows;
             HIPCHK(c, hipMemcpyAsync(c->h_out, c->d_out,
                                      one_trip ? packed_bytes((size_t)nt) + full_bytes
                                               : sums_bytes + (size_t)nt * sizeof(int),

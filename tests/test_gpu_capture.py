@@ -87,3 +87,59 @@ def test_replays_between_other_calls(n, nt, prec):
             assert same(c.fetch(), want[1, i])
             c.upload(js[0].m, js[0].x, js[0].v, js[0].r2)
         g.free()
+
+
+@pytest.mark.parametrize("prec", [regf.PREC_SPLIT, regf.PREC_CHECKED])
+@pytest.mark.parametrize("n", [1024, 20000])
+def test_first_launch_of_a_context_recorded(n, prec):
+    """A block's first launch allocates nothing, so it can be recorded."""
+    say(f"case: first launch recorded n={n} precision={prec}")
+    js = workloads.plummer_kroupa(n, seed=3, k_nb=30)
+    rng = np.random.default_rng(n)
+    with regf.Context(device=0, cap=64, precision=prec) as c, \
+            regf.Context(device=0, cap=64, precision=prec) as d:
+        for k in (c, d):
+            k.upload(js.m, js.x, js.v, js.r2)
+        c.set_targets(rng.permutation(n)[:16].astype(np.int32))
+        g = Graph(c)
+        with g:
+            c.launch()
+        for _ in range(3):
+            t = rng.permutation(n)[:16].astype(np.int32)
+            c.set_targets(t)
+            g.replay()
+            assert same(c.fetch(), d.query(t))
+        g.free()
+
+
+@pytest.mark.parametrize("prec", [regf.PREC_SPLIT, regf.PREC_CHECKED])
+@pytest.mark.parametrize("n", [1024, 20000])
+def test_replay_after_a_query_of_more_rows(n, prec):
+    """Queries of up to 4096 targets within the context's capacity, also with
+    more than 1 MB of list rows, leave the buffers of a recorded launch of 16
+    targets where they are."""
+    say(f"case: replay after larger queries n={n} precision={prec}")
+    js = workloads.plummer_kroupa(n, seed=4, k_nb=30)
+    rng = np.random.default_rng(n)
+    sizes = (min(n, 4096), 900, min(n, 2500), 64)
+    with regf.Context(device=0, cap=400, precision=prec) as c, \
+            regf.Context(device=0, cap=400, precision=prec) as d:
+        for k in (c, d):
+            k.upload(js.m, js.x, js.v, js.r2)
+        # the scratch and outputs of every block, before anything is recorded
+        for nt in sizes:
+            c.set_targets(np.arange(nt, dtype=np.int32))
+            c.launch()
+            c.fetch()
+        c.set_targets(rng.permutation(n)[:16].astype(np.int32))
+        g = Graph(c)
+        with g:
+            c.launch()
+        for nt in sizes[1:] + sizes[:1]:
+            big = rng.permutation(n)[:nt].astype(np.int32)
+            assert same(c.query(big), d.query(big))
+            t = rng.permutation(n)[:16].astype(np.int32)
+            c.set_targets(t)
+            g.replay()
+            assert same(c.fetch(), d.query(t))
+        g.free()
