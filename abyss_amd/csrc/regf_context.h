@@ -194,4 +194,7 @@ int ctx_set_targets(abyss_ctx_t c, int nt, const int *targets, TargetWait wait);
 int ctx_wait(abyss_ctx_t c);
 // Whether a caller's capture is recording the context's stream.
 int ctx_capturing(abyss_ctx_t c, bool *capturing);
+// ABYSS_ERR_HIP under such a capture: for a call that waits for the stream, but
+// not before it has enqueued work or changed what the context holds.
+int refuse_capture(abyss_ctx_t c);
 }  // namespace abyss

@@ -402,7 +402,9 @@ int abyss_ctx_irregular(abyss_ctx_t c, int nt, const int *targets, double *acc, 
             return ABYSS_ERR_TARGET_RANGE;
         }
     if (hipSetDevice(c->device) != hipSuccess) return ABYSS_ERR_HIP;
-    int rc = ensure_resident_lists(c);   // a j-set of another size: empty lists
+    int rc = abyss::refuse_capture(c);
+    if (rc != ABYSS_OK) return rc;
+    rc = ensure_resident_lists(c);   // a j-set of another size: empty lists
     if (rc != ABYSS_OK) return rc;
     if (c->busy_irr && (rc = abyss::ctx_wait(c)) != ABYSS_OK) return rc;
     // targets in (read in place up to kMappedListTargets), results straight

@@ -982,6 +982,14 @@ int ctx_capturing(abyss_ctx_t c, bool *capturing)
     return ABYSS_OK;
 }
 
+int refuse_capture(abyss_ctx_t c)
+{
+    bool capturing = false;
+    int rc = ctx_capturing(c, &capturing);
+    if (rc != ABYSS_OK || !capturing) return rc;
+    return set_detail(c, ABYSS_ERR_HIP, "a call that waits for its results cannot be recorded");
+}
+
 // The previous launch may still read the target list and write the outputs.
 // With TargetWait::kUse an upload or a prediction is not waited for, so that
 // the launch is queued by the time they end.  N = 65536: upload and query of
@@ -1002,6 +1010,7 @@ int ctx_set_targets(abyss_ctx_t c, int nt, const int *targets, TargetWait wait)
                               targets[k], c->n);
     HIPCHK(c, hipSetDevice(c->device));
     int rc = ABYSS_OK;
+    if (wait == TargetWait::kUse && (rc = refuse_capture(c)) != ABYSS_OK) return rc;
     if (wait == TargetWait::kStream ||
         (wait == TargetWait::kUse &&
          (c->busy_tgt || (size_t)nt > c->t_capacity || (!c->closed && c->tgt == c->h_tgt_dev))))

@@ -200,10 +200,8 @@ int abyss_ctx_update_state(abyss_ctx_t c, int count, const int *idx, const doubl
     }
     if (hipSetDevice(c->device) != hipSuccess) return ABYSS_ERR_HIP;
     // a captured update would read whatever the staging holds at its replays
-    bool capturing = false;
-    int rc = abyss::ctx_capturing(c, &capturing);
+    int rc = abyss::refuse_capture(c);
     if (rc != ABYSS_OK) return rc;
-    if (capturing) return ABYSS_ERR_HIP;
     // staging from a previous update may still be in flight
     if (c->busy_upd) {
         rc = abyss::ctx_wait(c);

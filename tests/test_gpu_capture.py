@@ -143,3 +143,42 @@ def test_replay_after_a_query_of_more_rows(n, prec):
             g.replay()
             assert same(c.fetch(), d.query(t))
         g.free()
+
+
+def test_calls_that_wait_are_refused_and_leave_nothing_behind():
+    """Under a capture the calls that wait for their results, and updates of the
+    state, fail; the capture goes on, and the context holds what it held."""
+    say("case: calls refused under a capture")
+    n, cap = 5000, 128
+    js = workloads.plummer_kroupa(n, seed=5, k_nb=30)
+    rng = np.random.default_rng(5)
+    a, ad = 0.1 * rng.normal(size=(n, 3)), 0.1 * rng.normal(size=(n, 3))
+    t, other = (rng.permutation(n)[:300].astype(np.int32) for _ in range(2))
+    dt, a_old = np.full(300, 1e-3), np.zeros((300, 6))
+    with regf.Context(device=0, cap=cap) as c, regf.Context(device=0, cap=cap) as d:
+        for k in (c, d):
+            k.upload_state(js.m, js.x, js.v, a, ad, np.zeros(n), js.r2)
+            k.keep_lists()
+            k.query(np.arange(n, dtype=np.int32))
+            k.irregular(t)
+            # gather records of the positions before, not of these
+            k.upload_state(js.m, 1.01 * js.x, js.v, a, ad, np.zeros(n), js.r2)
+        held = [p.copy() for p in c.query(t)]
+        d.query(t)
+        g = Graph(c)
+        with g:
+            for call in (lambda: c.query(other), lambda: c.irregular(other),
+                         lambda: c.regular_step(other, dt, a_old),
+                         lambda: c.update_state(other, js.m[other], 2 * js.x[other], js.v[other],
+                                                a[other], ad[other], np.zeros(300),
+                                                js.r2[other])):
+                with pytest.raises(regf.AbyssError) as e:
+                    call()
+                assert e.value.code == regf.ERR_HIP
+        assert same(c.fetch(), held)
+        assert same(c.irregular(t), d.irregular(t))
+        for k in (c, d):
+            k.predict(2.0 ** -7)
+        assert same(c.irregular(other), d.irregular(other))
+        assert same(c.regular_step(other, dt, a_old), d.regular_step(other, dt, a_old))
+        g.free()
