@@ -41,6 +41,8 @@ struct abyss_ctx_s {
     // replay at any time between calls: calls then keep to the buffers and the
     // waits that such work can rely on (ctx_launch_force, ctx_set_targets).
     bool captured = false;
+    // ... has recorded a prediction, so the j-set may change with no call
+    bool predict_recorded = false;
     int *d_tgt = nullptr, *h_tgt = nullptr;
     // h_tgt is mapped, coherent pinned memory; h_tgt_dev is its device
     // address.  `tgt` is the target array the kernels read: h_tgt_dev for

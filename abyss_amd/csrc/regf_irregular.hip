@@ -297,11 +297,12 @@ int ensure_resident_lists(abyss_ctx_t c)
 }
 
 // The AoS gather copy of the current j-set (rebuilt after an upload or a
-// prediction).
+// prediction, and for every call once a caller may replay predictions).
 int ensure_aos(abyss_ctx_t c)
 {
     const size_t need = (size_t)c->n * sizeof(JRec);
-    if (c->aos_version == c->jset_version && c->aos_bytes >= need) return ABYSS_OK;
+    if (!c->predict_recorded && c->aos_version == c->jset_version && c->aos_bytes >= need)
+        return ABYSS_OK;
     if (need > c->aos_bytes) {
         if (hipStreamSynchronize(c->stream) != hipSuccess) return ABYSS_ERR_HIP;
         if (c->d_aos) (void)hipFree(c->d_aos);

@@ -258,11 +258,16 @@ int abyss_ctx_predict(abyss_ctx_t c, double t_new)
     const int n = c->state_n;
     double *jx = reinterpret_cast<double *>(c->d_j);
     float *m32 = reinterpret_cast<float *>(jx + 8 * (size_t)n);
+    bool capturing = false;
+    int rc = abyss::ctx_capturing(c, &capturing);
+    if (rc != ABYSS_OK) return rc;
     // with resident lists in use, their gather records come from the same
-    // pass (a pack of their own otherwise: 5 us at N = 65536)
-    abyss::JRec *aos = c->keep_lists && c->aos_bytes >= (size_t)n * sizeof(abyss::JRec)
-                           ? reinterpret_cast<abyss::JRec *>(c->d_aos)
-                           : nullptr;
+    // pass (a pack of their own otherwise: 5 us at N = 65536); not when it is
+    // being recorded, since nobody knows whether and when it will run
+    if (capturing) c->predict_recorded = true;
+    const bool records =
+        !capturing && c->keep_lists && c->aos_bytes >= (size_t)n * sizeof(abyss::JRec);
+    abyss::JRec *aos = records ? reinterpret_cast<abyss::JRec *>(c->d_aos) : nullptr;
     hipLaunchKernelGGL(predict_kernel, dim3((n + 255) / 256), dim3(256), 0, c->stream,
                        state_view(c->d_state, n), n, t_new, jx, m32, aos);
     c->jset_version += 1;

@@ -182,3 +182,34 @@ def test_calls_that_wait_are_refused_and_leave_nothing_behind():
         assert same(c.irregular(other), d.irregular(other))
         assert same(c.regular_step(other, dt, a_old), d.regular_step(other, dt, a_old))
         g.free()
+
+
+def test_recorded_predictions_and_the_irregular_force():
+    """A prediction that is recorded but not run leaves the j-set, and what the
+    irregular force reads of it, as uploaded; each replay moves both."""
+    say("case: recorded predictions")
+    n, t_new = 5000, 2.0 ** -6
+    js = workloads.plummer_kroupa(n, seed=7, k_nb=30)
+    rng = np.random.default_rng(7)
+    a, ad = 0.1 * rng.normal(size=(n, 3)), 0.1 * rng.normal(size=(n, 3))
+    t = rng.permutation(n)[:500].astype(np.int32)
+    with regf.Context(device=0, cap=128) as c, regf.Context(device=0, cap=128) as d:
+        for k in (c, d):
+            k.upload_state(js.m, js.x, js.v, a, ad, np.zeros(n), js.r2)
+            k.keep_lists()
+            k.query(np.arange(n, dtype=np.int32))
+            k.irregular(t)
+            # gather records of the positions before, not of these
+            k.upload_state(js.m, 1.01 * js.x, js.v, a, ad, np.zeros(n), js.r2)
+        g = Graph(c)
+        with g:
+            c.predict(t_new)
+        assert same(c.irregular(t), d.irregular(t))
+        for factor in (1.01, 1.02):
+            g.replay()
+            d.predict(t_new)
+            assert same(c.irregular(t), d.irregular(t))
+            for k in (c, d):
+                k.upload_state(js.m, factor * js.x, js.v, a, ad, np.zeros(n), js.r2)
+            assert same(c.irregular(t), d.irregular(t))
+        g.free()
