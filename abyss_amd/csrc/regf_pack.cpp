@@ -14,6 +14,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <condition_variable>
 #include <functional>
 #include <mutex>
@@ -23,8 +24,7 @@
 namespace abyss {
 namespace {
 
-// Parts [1, parts) of a job run on parked worker threads, part 0 on the
-// caller; run() returns when every part is done.  One job at a time: a
+// Parts [1, parts) of a job run on worker threads, part 0 on the caller; run() returns when every part is done.  One job at a time: a
 // caller that finds the pool busy does the whole job itself.
 class Pool {
 public:
@@ -63,6 +63,7 @@ public:
         }
         cv_.notify_all();
         f(0);
+        linger([this] { return left_ == 0; });
         std::unique_lock<std::mutex> lk(mu_);
         done_cv_.wait(lk, [this] { return left_ == 0; });
         job_ = nullptr;
@@ -71,6 +72,18 @@ public:
 
 private:
     static constexpr unsigned kMaxWorkers = 7;
+    // After a job a worker looks for the next one this long before it parks,
+    // and the caller for its workers' end: pieces of a result arrive 40 us
+    // apart, and waking a parked thread takes 10 to 20 us.  Results of 32
+    // clusters 3450 us without, 3270 with 50 us; 30011 targets 1081, 1065.
+    static constexpr std::chrono::microseconds kLinger{50};
+
+    template <class F>
+    static void linger(const F &until)
+    {
+        const auto end = std::chrono::steady_clock::now() + kLinger;
+        while (!until() && std::chrono::steady_clock::now() < end) std::this_thread::yield();
+    }
 
     void loop(int part)
     {
@@ -86,8 +99,11 @@ private:
                 f = job_;
             }
             (*f)(part);
-            std::lock_guard<std::mutex> lk(mu_);
-            if (--left_ == 0) done_cv_.notify_one();
+            {
+                std::lock_guard<std::mutex> lk(mu_);
+                if (--left_ == 0) done_cv_.notify_one();
+            }
+            linger([&] { return gen_ != seen; });
         }
     }
 
@@ -97,8 +113,9 @@ private:
     std::mutex mu_;
     std::condition_variable cv_, done_cv_;
     const std::function<void(int)> *job_ = nullptr;
-    int parts_ = 0, left_ = 0;
-    long long gen_ = 0;
+    int parts_ = 0;
+    std::atomic<int> left_{0};          // written under mu_
+    std::atomic<long long> gen_{0};     // written under mu_
     bool stop_ = false;
 };
 
@@ -238,6 +255,20 @@ PackStatus pack_jset(int n, int j0, int j1, const double *m, const double *x, co
 int host_parts() { return pool().workers() + 1; }
 
 bool host_run(int parts, const std::function<void(int)> &f) { return pool().run(parts, f); }
+
+bool copy_arriving(int steps, int parts, const std::function<bool(int)> &wait,
+                   const std::function<bool(int)> &here,
+                   const std::function<void(int, int, int, int)> &copy)
+{
+    for (int k0 = 0, k1 = 0; k0 < steps; k0 = k1) {
+        if (!wait(k0)) return false;
+        for (k1 = k0 + 1; k1 < steps && here(k1);) ++k1;
+        const auto job = [&](int p) { copy(k0, k1, p, parts); };
+        // by reference: the function object must not allocate
+        if (parts <= 1 || !host_run(parts, std::ref(job))) copy(k0, k1, 0, 1);
+    }
+    return true;
+}
 
 void unpack_rows(int k0, int k1, const int *counts, const int *rows, size_t stride, int cap,
                  int *list)

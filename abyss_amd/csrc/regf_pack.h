@@ -43,6 +43,15 @@ int host_parts();
 // run, when another caller's job holds the pool.
 bool host_run(int parts, const std::function<void(int)> &f);
 
+// Copies `steps` pieces that arrive one after the other: wait(k) returns once
+// piece k is there (false: it will not be), here(k) tells without waiting, and
+// copy(k0, k1, p, parts) copies part p of the pieces [k0, k1).  Only the
+// calling thread waits, and the pool is free meanwhile: a job on up to `parts`
+// threads copies the pieces that have arrived.  False when a wait failed.
+bool copy_arriving(int steps, int parts, const std::function<bool(int)> &wait,
+                   const std::function<bool(int)> &here,
+                   const std::function<void(int, int, int, int)> &copy);
+
 // Copies the populated entries (min(|counts[k]|, cap)) of list rows [k0, k1)
 // from `rows` (row stride `stride`) to `list` (row stride cap).
 void unpack_rows(int k0, int k1, const int *counts, const int *rows, size_t stride, int cap,

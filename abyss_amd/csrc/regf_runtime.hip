@@ -21,9 +21,8 @@
 #include <string.h>
 
 #include <algorithm>
-#include <atomic>
+#include <functional>
 #include <mutex>
-#include <thread>
 
 using abyss::JState;
 using abyss::Plan;
@@ -1268,65 +1267,57 @@ namespace abyss {
 
 namespace {
 
-// Copies the host block's acc, adot and counts and the list rows into the
+// Copies the host block's counts, acc and adot and the list rows into the
 // caller's arrays; with chunks > 0 the rows of chunk k are there once
 // c->fev[k] has completed, with sums_late acc and adot, after the rows, once
 // c->sums_ev has.  Large results are copied by several host threads, each a
-// slice of every chunk: one waits for the events and lets the others (and
-// itself) at the chunks that have arrived.
+// slice of what has arrived; the threads are asked for only then, so that
+// neither they nor another context's upload or fetch wait for this GPU's work.
 hipError_t unpack_results(abyss_ctx_t c, int chunks, bool sums_late, const int *rows,
                           size_t stride, size_t list_bytes, double *acc, double *adot, int *nnb,
                           int *list)
 {
     const int nt = c->nt, cap = c->cap;
     const int nchunk = std::max(chunks, 1);
-    const int steps = nchunk + (sums_late ? 1 : 0);   // the last: acc and adot
-    std::atomic<int> ready{chunks > 0 ? 0 : nchunk};
-    hipError_t err = hipSuccess;   // written by part 0 before it opens the last step
-    int parts = 1;
-    const auto part = [&](int p) {
+    const int last = nchunk + (sums_late ? 1 : 0);
+    hipError_t err = hipSuccess;
+    // pieces: 0 what the host block has, then the chunks of rows, then acc and
+    // adot if they come late; a piece without an event is here from the start
+    const auto event = [&](int k) -> hipEvent_t {
+        if (k == 0 || (k <= nchunk && chunks == 0)) return nullptr;
+        return k <= nchunk ? c->fev[k - 1] : c->sums_ev;
+    };
+    const auto wait = [&](int k) {
+        if (event(k)) err = hipEventSynchronize(event(k));
+        return err == hipSuccess;
+    };
+    const auto here = [&](int k) {
+        if (!event(k) || hipEventQuery(event(k)) == hipSuccess) return true;
+        (void)hipGetLastError();   // "not ready" is no error of a later launch
+        return false;
+    };
+    const auto copy = [&](int k0, int k1, int p, int parts) {
         const auto slice = [&](int a, int b, int *lo, int *hi) {
             *lo = a + (int)((long long)(b - a) * p / parts);
             *hi = a + (int)((long long)(b - a) * (p + 1) / parts);
         };
-        // false: a wait failed, nothing more arrives
-        const auto arrived = [&](int k) {
-            if (p == 0 && ready.load(std::memory_order_relaxed) <= k) {
-                err = hipEventSynchronize(k < nchunk ? c->fev[k] : c->sums_ev);
-                ready.store(err == hipSuccess ? k + 1 : -1, std::memory_order_release);
-            }
-            int r = ready.load(std::memory_order_acquire);
-            while (r >= 0 && r <= k) {
-                std::this_thread::yield();
-                r = ready.load(std::memory_order_acquire);
-            }
-            return r >= 0;
-        };
-        const auto sums = [&]() {
-            int lo = 0, hi = 0;
-            slice(0, nt, &lo, &hi);
+        int lo = 0, hi = 0;
+        slice(0, nt, &lo, &hi);
+        if (k0 == 0) memcpy(nnb + lo, c->h_nnb + lo, (size_t)(hi - lo) * sizeof(int));
+        if (sums_late ? k1 > last : k0 == 0) {
             const size_t n3 = 3 * (size_t)(hi - lo), o3 = 3 * (size_t)lo;
             memcpy(acc + o3, c->h_res + o3, n3 * sizeof(double));
             memcpy(adot + o3, c->h_res + 3 * (size_t)nt + o3, n3 * sizeof(double));
-        };
-        int lo = 0, hi = 0;
-        slice(0, nt, &lo, &hi);
-        memcpy(nnb + lo, c->h_nnb + lo, (size_t)(hi - lo) * sizeof(int));
-        if (!sums_late) sums();
-        for (int k = 0; k < nchunk; ++k) {
-            if (!arrived(k)) return;
-            slice((int)((long long)nt * k / nchunk), (int)((long long)nt * (k + 1) / nchunk), &lo,
-                  &hi);
-            abyss::unpack_rows(lo, hi, c->h_nnb, rows, stride, cap, list);
         }
-        if (steps > nchunk && arrived(nchunk)) sums();
+        const int r0 = std::max(k0 - 1, 0), r1 = std::min(k1 - 1, nchunk);
+        if (r0 >= r1) return;
+        slice((int)((long long)nt * r0 / nchunk), (int)((long long)nt * r1 / nchunk), &lo, &hi);
+        abyss::unpack_rows(lo, hi, c->h_nnb, rows, stride, cap, list);
     };
-    if (list_bytes >= kUnpackParallelBytes) {
-        parts = std::min(abyss::host_parts(), kUnpackParts);
-        if (parts > 1 && abyss::host_run(parts, part)) return err;
-        parts = 1;
-    }
-    part(0);
+    const int parts = list_bytes >= kUnpackParallelBytes
+                          ? std::min(abyss::host_parts(), kUnpackParts)
+                          : 1;
+    abyss::copy_arriving(last + 1, parts, std::ref(wait), std::ref(here), std::ref(copy));
     return err;
 }
 
