@@ -191,7 +191,16 @@ __global__ __launch_bounds__(256) void irregular_kernel(const JRec *__restrict__
 // out row (18): x_new, v_new, a2, a3, a_irr, adot_irr.
 // STAGED: both lists of the wave's target are first copied into LDS
 // (dynamic, 2 * cap ints per wave), so the membership binary searches read
-// LDS instead of paying global-memory latency at every step.
+// LDS instead of paying global-memory latency at every step.  The wave's
+// part of the dynamic LDS (correct_lds_ints) then takes the target's results,
+// which go out in one run.
+constexpr int kCorrectRow = 18;   // doubles of an out row
+__host__ __device__ constexpr int correct_lds_ints(bool staged, int cap)
+{
+    const int row = kCorrectRow * (int)(sizeof(double) / sizeof(int));
+    return staged && 2 * cap > row ? 2 * cap : row;
+}
+
 template <bool STAGED>
 __global__ __launch_bounds__(256) void correct_kernel(
     const JRec *__restrict__ jr, const int *__restrict__ tgt, int nt, const int *__restrict__ new_nnb,
@@ -200,8 +209,9 @@ __global__ __launch_bounds__(256) void correct_kernel(
     const int *__restrict__ rlist, const double *__restrict__ dts,
     const double *__restrict__ a_old, double *__restrict__ out)
 {
-    extern __shared__ int s_lists[];   // STAGED: [4 waves][new cap | old cap]
-    __shared__ double s_row[4][18];    // a target's results, written out in one run
+    // [4 waves][new cap | old cap (STAGED), then the row]
+    extern __shared__ double s_lds[];
+    double *mine = s_lds + (threadIdx.x >> 6) * (correct_lds_ints(STAGED, cap) / 2);
     const int lane = threadIdx.x & 63;
     const int q = blockIdx.x * 4 + (threadIdx.x >> 6);
     const bool active = q < nt;
@@ -211,7 +221,7 @@ __global__ __launch_bounds__(256) void correct_kernel(
     const int *ln = new_list + (size_t)q * cap;
     const int *lo = rlist + (size_t)i * cap;
     if constexpr (STAGED) {
-        int *sn = s_lists + (threadIdx.x >> 6) * 2 * cap;
+        int *sn = reinterpret_cast<int *>(mine);
         int *so = sn + cap;
         for (int e = lane; e < cn; e += 64) sn[e] = ln[e];
         for (int e = lane; e < co; e += 64) so[e] = lo[e];
@@ -249,7 +259,11 @@ __global__ __launch_bounds__(256) void correct_kernel(
         }
     }
     wave_sum<12>(a);
-    double *row = s_row[threadIdx.x >> 6];
+    // the wave has read its lists
+    double *row = mine;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     if (lane < 3) {
         // selects, not a lane-indexed array
         const double a1 = new_acc[(size_t)q * 3 + d], j1 = new_adot[(size_t)q * 3 + d];
@@ -269,7 +283,7 @@ __global__ __launch_bounds__(256) void correct_kernel(
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (lane < 18) out[(size_t)q * 18 + lane] = row[lane];
+    if (lane < kCorrectRow) out[(size_t)q * kCorrectRow + lane] = row[lane];
 }
 
 #pragma clang fp contract(on)
@@ -492,15 +506,16 @@ int abyss_ctx_regular_step(abyss_ctx_t c, int nt, const int *targets, const doub
     rc = ensure_aos(c);
     if (rc != ABYSS_OK) return rc;
     // lists staged in LDS when both fit (2 * cap ints per wave, 64 KB per
-    // workgroup at most)
-    const size_t lds = 4 * 2 * (size_t)c->cap * sizeof(int);
-    if (lds <= 65536)
+    // workgroup at most: a stride of up to 2048)
+    const bool staged = c->cap <= 2048;
+    const size_t lds = 4 * (size_t)correct_lds_ints(staged, c->cap) * sizeof(int);
+    if (staged)
         hipLaunchKernelGGL(correct_kernel<true>, dim3((nt + 3) / 4), dim3(256), lds, c->stream,
                            reinterpret_cast<const JRec *>(c->d_aos), c->tgt, nt, c->d_nnb,
                            c->d_list, c->d_acc, c->d_adot, c->cap, rnnb, rlist, d_in, d_in + nt,
                            d_out);
     else
-        hipLaunchKernelGGL(correct_kernel<false>, dim3((nt + 3) / 4), dim3(256), 0, c->stream,
+        hipLaunchKernelGGL(correct_kernel<false>, dim3((nt + 3) / 4), dim3(256), lds, c->stream,
                            reinterpret_cast<const JRec *>(c->d_aos), c->tgt, nt, c->d_nnb,
                            c->d_list, c->d_acc, c->d_adot, c->cap, rnnb, rlist, d_in, d_in + nt,
                            d_out);

@@ -365,3 +365,33 @@ def test_one_split_at_the_scratch_limit(prec):
             assert c.plan()["j_splits"] == 1
     for p, q in zip(*out):
         assert np.array_equal(p, q)
+
+
+@pytest.mark.parametrize("cap", [1, 17, 18, 700, 2030, 2031, 2048, 2049])
+def test_regular_step_around_the_staged_lists(cap):
+    """The corrector stages the old and new list of a target in LDS when both
+    fit the workgroup's share, where the target's results follow them; lists of
+    other strides are read where they are: the same bytes, and the irregular
+    force of the step is that over the new lists, also overflowed ones."""
+    say(f"case: staged lists cap={cap}")
+    n, m = 4000, 70
+    js = workloads.plummer_kroupa(n, seed=11, k_nb=300)
+    rng = np.random.default_rng(11)
+    t = rng.permutation(n)[:m].astype(np.int32)
+    dt, a_old = rng.uniform(1e-3, 1e-2, m), rng.normal(size=(m, 6))
+    z, out = np.zeros((n, 3)), []
+    for stride in (cap, 701):
+        with regf.Context(device=0, cap=stride) as c:
+            c.upload_state(js.m, js.x, js.v, z, z, np.zeros(n), js.r2)
+            c.keep_lists()
+            c.query(t)
+            c.predict(2.0 ** -5)   # other neighbours
+            out.append(c.regular_step(t, dt, a_old))
+            acc, adot = c.irregular(t)
+            assert np.array_equal(out[-1][4][:, 12:15], acc)
+            assert np.array_equal(out[-1][4][:, 15:], adot)
+    if cap < 700:
+        return
+    for k in (0, 1, 2, 4):
+        assert np.array_equal(out[0][k], out[1][k])
+    assert np.array_equal(out[0][3][:, :700], out[1][3][:, :700]) and (out[0][2] > 0).all()
