@@ -38,13 +38,18 @@ public:
         for (auto &t : th_) t.join();
     }
 
-    // Workers available to a job (0: the pool could not start).
+    // Workers available to a job: as many as could be started (0: none).
     int workers()
     {
         std::call_once(once_, [this] {
             const unsigned hw = std::thread::hardware_concurrency();
             const int want = (int)std::min<unsigned>(kMaxWorkers, hw > 1 ? hw - 1 : 0);
-            for (int k = 0; k < want; ++k) th_.emplace_back([this, k] { loop(k + 1); });
+            try {
+                for (int k = 0; k < want; ++k) th_.emplace_back([this, k] { loop(k + 1); });
+            } catch (...) {
+                // no memory or no more threads for this process: the calls,
+                // whose entries are C, go on with those that run
+            }
         });
         return (int)th_.size();
     }

@@ -1,9 +1,11 @@
 // Copies of results that arrive in pieces (regf_pack.cpp), built and run by
 // tests/test_copy_cpu.py: every piece is copied once and only after it has
 // arrived, and the pool takes another caller's job while a copy waits.
-//   copy_check pieces | pool
+//   copy_check pieces | pool | few
+// few: the process may start a few threads only; a job runs on those.
 #include <stdio.h>
 #include <string.h>
+#include <sys/resource.h>
 
 #include <algorithm>
 #include <functional>
@@ -74,11 +76,26 @@ static void pool()
     CHECK(taken == 4);
 }
 
+static void few()
+{
+    // address space for the stacks of a few threads
+    struct rlimit lim;
+    CHECK(getrlimit(RLIMIT_AS, &lim) == 0);
+    lim.rlim_cur = 40u << 20;
+    CHECK(setrlimit(RLIMIT_AS, &lim) == 0);
+    const int parts = abyss::host_parts();
+    CHECK(parts >= 1 && parts <= 8);
+    std::vector<int> ran(8, 0);
+    CHECK(abyss::host_run(parts, [&](int p) { ran[p] += 1; }));
+    for (int p = 0; p < 8; ++p) CHECK(ran[p] == (p < parts ? 1 : 0));
+}
+
 int main(int argc, char **argv)
 {
     const char *what = argc > 1 ? argv[1] : "";
     if (!strcmp(what, "pieces")) pieces();
     else if (!strcmp(what, "pool")) pool();
+    else if (!strcmp(what, "few")) few();
     else return 2;
     printf("OK: %d failure(s)\n", fails);
     return fails ? 1 : 0;

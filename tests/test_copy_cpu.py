@@ -29,3 +29,12 @@ def test_copies_of_arriving_pieces(driver, what):
                        env=dict(os.environ, TSAN_OPTIONS="halt_on_error=1"))
     print(p.stdout[-1000:], p.stderr[-2000:])
     assert p.returncode == 0 and "OK: 0 failure(s)" in p.stdout
+
+
+def test_pool_of_a_process_that_cannot_start_more_threads(tmp_path):
+    exe = str(tmp_path / "copy_check")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-g", "-pthread", DRIVER, PACK, "-o", exe],
+                   check=True)
+    p = subprocess.run([exe, "few"], capture_output=True, text=True, timeout=100)
+    print(p.stdout[-1000:], p.stderr[-2000:])
+    assert p.returncode == 0 and "OK: 0 failure(s)" in p.stdout
