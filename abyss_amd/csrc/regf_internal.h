@@ -244,10 +244,9 @@ hipError_t launch_check_flag(const double *acc, const double *adot, const float 
                              const int *tgt, int nt, double k2, int *counters, int *fq, int *fi,
                              hipStream_t st);
 // Sums the recomputation's S partials of each of the m flagged targets (in
-// split order) and writes them over acc/adot (and the mirror's) at fq[k].
+// split order) and writes them over acc/adot at fq[k].
 hipError_t launch_recheck_finalize(const QueryOut &part, int S, int m, const int *fq,
-                                   double *acc, double *adot, const FinalMirror &mirror,
-                                   hipStream_t st);
+                                   double *acc, double *adot, hipStream_t st);
 // The recomputation of the first *count targets of fi (count on the device,
 // at most nt): `grid` workgroups loop over the (target block, split) items of
 // plan p (lanes per target, splits and span; 256-record tiles, 4 waves), then

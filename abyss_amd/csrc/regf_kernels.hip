@@ -1767,11 +1767,10 @@ hipError_t launch_pack_rows(const int *list, const int *nnb, int cap, int q0, in
 }
 
 hipError_t launch_recheck_finalize(const QueryOut &part, int S, int m, const int *fq,
-                                   double *acc, double *adot, const FinalMirror &mirror,
-                                   hipStream_t st)
+                                   double *acc, double *adot, hipStream_t st)
 {
     hipLaunchKernelGGL(recheck_finalize_kernel, dim3((m + 3) / 4), dim3(256), 0, st, part, S, m,
-                       m, (const int *)nullptr, (int *)nullptr, fq, acc, adot, mirror);
+                       m, (const int *)nullptr, (int *)nullptr, fq, acc, adot, FinalMirror{});
     return hipGetLastError();
 }
 

@@ -24,8 +24,9 @@
 namespace abyss {
 namespace {
 
-// Parts [1, parts) of a job run on worker threads, part 0 on the caller; run() returns when every part is done.  One job at a time: a
-// caller that finds the pool busy does the whole job itself.
+// Parts [1, parts) of a job run on worker threads, part 0 on the caller; run()
+// returns when every part is done.  One job at a time: a caller that finds the
+// pool busy does the whole job itself.
 class Pool {
 public:
     ~Pool()

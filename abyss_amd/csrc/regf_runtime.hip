@@ -549,7 +549,7 @@ int send_rows(abyss_ctx_t c, hipStream_t st, int groups)
 
 // The recomputation of m flagged targets (c->chk_fq / chk_fi hold them),
 // planned for m; the stream need not be idle.
-int recompute_flagged(abyss_ctx_t c, int m, const abyss::FinalMirror &mirror)
+int recompute_flagged(abyss_ctx_t c, int m)
 {
     c->n_rechecked = m;
     if (m <= 0) return ABYSS_OK;
@@ -561,7 +561,7 @@ int recompute_flagged(abyss_ctx_t c, int m, const abyss::FinalMirror &mirror)
     HIPCHK(c, abyss::launch_regf(c->js, c->chk_fi, m, rp, rpart, 0, abyss::kPrecRecheck,
                                  c->stream));
     HIPCHK(c, abyss::launch_recheck_finalize(rpart, rp.splits, m, c->chk_fq, c->d_acc, c->d_adot,
-                                             mirror, c->stream));
+                                             c->stream));
     return ABYSS_OK;
 }
 
@@ -594,8 +594,9 @@ Plan plan_recheck_loop(abyss_ctx_t c, int nt, int n, int max_splits, int *grid)
 // flagged them: `flagged`) and recomputes them with FP64 terms over the
 // same regular set: the flagged count is read back (a host wait) and the
 // recomputation planned for it.  (Blocks small enough to skip that wait run
-// in FP64 terms in one pass instead, Plan::fp64_terms.)  The recomputed
-// targets' results also go to the mirror when it is set.  rows_early: a fetch
+// in FP64 terms in one pass instead, Plan::fp64_terms.)  The mirror, when set,
+// gets the recomputed targets' results too; only blocks whose flagged count
+// stays on the device have one.  rows_early: a fetch
 // follows, and the list rows, which the recomputation leaves as they are,
 // start on their way to the host beside it.  King N = 262144, every target
 // (recomputation 4.9 ms, rows 2.2 ms): query 60.1 -> 56.6 ms; N = 65536, 20011
@@ -626,10 +627,13 @@ int recheck(abyss_ctx_t c, bool flagged, const abyss::FinalMirror &mirror, bool 
         c->recheck_pending = true;
         return ABYSS_OK;
     }
+    // the merge of a larger block writes no mirror, so that the recomputation
+    // need not either
+    static_assert(kQueryMirrorTargets <= abyss::kRecheckOnDeviceMax, "mirrored blocks end above");
     HIPCHK(c, hipMemcpyAsync(c->h_chk, c->chk_counters, sizeof(int), hipMemcpyDeviceToHost,
                              c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    int rc = recompute_flagged(c, c->h_chk[0], mirror);
+    int rc = recompute_flagged(c, c->h_chk[0]);
     if (rc != ABYSS_OK || !rows_early) return rc;
     // the merge has finished, so the side stream need not wait for it
     if (!c->side) HIPCHK(c, hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
