@@ -625,7 +625,11 @@ __device__ __forceinline__ void jl4_list(JLLane &L, NearMask m, int count, int j
 // A tile of TILE records for four lanes per target in FP32 terms (TM 0),
 // `count` of them valid (FULL: all; the rest zero-filled, mass 0).  The
 // pairs, the grouped neighbour test and the order of every sum are those of
-// jl_tile_common and jl_tile.
+// jl_tile_common and jl_tile.  Wave priorities (PRIO of jl_tile_common) at any
+// span: beside the lists a workgroup of few tiles gains as well.  Force kernel,
+// N / targets, priorities from 8 tiles on -> always: 10007 / 10007 checked
+// 110.3 -> 108.3 us (3 tiles), 16385 / 4096 split 82 -> 79.7 us (3), 30000 /
+// 3000 checked 95.7 -> 93.5 us (3), 32768 / 8000 228.6 -> 225 us (4).
 template <bool FULL, int TILE>
 __device__ __forceinline__ void jl4_tile_fp32(JLLane &L, const double2 *__restrict__ pos,
                                               const float *__restrict__ mass, int count,
@@ -1310,8 +1314,8 @@ void recheck_kernel_loop(JState js, const int *__restrict__ tgt, const int *__re
     constexpr int TPB = 4 * (64 / JL);   // targets per workgroup
     const int items = (m + TPB - 1) / TPB * splits;
     for (int it = blockIdx.x; it < items; it += gridDim.x)
-        regf_body_jl<JL, 3, false, kTile, 4, JL == 4>(js, tgt, m, jspan, out, 0, 0, it / splits, it % splits, 0, nt_stride,
-                            s_pos, s_m);
+        regf_body_jl<JL, 3, false, kTile, 4, JL == 4>(js, tgt, m, jspan, out, 0, 0, it / splits,
+                                                      it % splits, 0, nt_stride, s_pos, s_m);
 }
 
 // One wave per flagged target k < m (m = *m_dev when m_dev is set; then
@@ -1352,15 +1356,22 @@ __global__ void batch_reset_kernel(int *counters)
 
 // One work item of a batch with the cluster's lanes per target and j-tile
 // in 4-wave workgroups: smaller tiles use the start of the LDS buffers.
+// Four lanes per target list by masks whatever the cluster's size: a batch has
+// no kernel of its own for a size, and a second body for clusters above
+// kMaskedMax costs every item registers.  One launch, before masks / with them
+// / with both bodies: 4 x 65536 all targets 15.6 / 14.0 / 15.7 ms, 131072 all
+// 16.8 / 14.0, 262144 all 53.0 / 51.9 / 54.3 ms, 8 x 40000 with 4000 2.66 /
+// 2.32 / 2.48 ms, 2 x 131072 with 30000 7.34 / 7.36 / 7.94 ms; the worst of
+// those measured, 2 x 131072 with 60000 checked: 13.95 / 14.2 ms.
 template <int JL, bool EST, int TILE>
 __device__ __forceinline__ void batch_body(const ClusterDesc &d, const WorkItem &w,
                                            const QueryOut &out, int cap, int fc,
                                            double2 (*s_pos)[kTile * 3], float (*s_m)[kTile])
 {
     regf_body_jl<JL, 0, EST, TILE, 4, JL == 4>(d.js, d.tgt, d.nt, d.jspan, out, cap, fc, w.tblock,
-                                      w.split, d.q_base, d.nt_stride,
-                                      reinterpret_cast<double2 (*)[TILE * 3]>(s_pos),
-                                      reinterpret_cast<float (*)[TILE]>(s_m));
+                                               w.split, d.q_base, d.nt_stride,
+                                               reinterpret_cast<double2 (*)[TILE * 3]>(s_pos),
+                                               reinterpret_cast<float (*)[TILE]>(s_m));
 }
 
 // Persistent: each workgroup takes work items from a device queue until it
@@ -1427,8 +1438,9 @@ void batch_recheck_kernel(const ClusterDesc *__restrict__ cd, const WorkItem *__
         const ClusterDesc &d = cd[w.cluster];
         switch (d.jl) {
             case 4:
-                regf_body_jl<4, 3, false, kTile, 4, true>(d.js, d.tgt, d.nt, d.jspan, d.part, 0, 0, w.tblock, w.split, 0,
-                                   d.nt, s_pos, s_m);
+                regf_body_jl<4, 3, false, kTile, 4, true>(d.js, d.tgt, d.nt, d.jspan, d.part, 0, 0,
+                                                          w.tblock, w.split, 0, d.nt, s_pos,
+                                                          s_m);
                 break;
             case 16:
                 regf_body_jl<16, 3>(d.js, d.tgt, d.nt, d.jspan, d.part, 0, 0, w.tblock, w.split,
@@ -1567,8 +1579,7 @@ TargetArg<JL> target_arg(const int *small, int nt)
 // Term mode 0 with the plan's shape (j-tile, wave64s per workgroup).
 template <int JL, bool EST, int TILE, int WPB>
 void launch_shape(const JState &js, const int *tgt, int nt, const Plan &p, const QueryOut &out,
-                  int cap, int fc, int *reset, const int *small,
-          hipStream_t st)
+                  int cap, int fc, int *reset, const int *small, hipStream_t st)
 {
     if constexpr (JL == 4) {
         if (js.n <= kMaskedMax) {
@@ -1583,7 +1594,7 @@ void launch_shape(const JState &js, const int *tgt, int nt, const Plan &p, const
                 hipLaunchKernelGGL((regf_kernel_jl<JL, 0, EST, TILE, WPB, false, true>),
                                    dim3(p.grid_x * p.splits), dim3(64 * WPB), 0, st, js, tgt, nt,
                                    p.jspan, out, cap, fc, reset, p.grid_x, p.splits,
-                               target_arg<JL>(small, nt));
+                                   target_arg<JL>(small, nt));
                 return;
             }
         }
@@ -1596,15 +1607,27 @@ void launch_shape(const JState &js, const int *tgt, int nt, const Plan &p, const
 template <int JL, bool EST>
 hipError_t launch_mode0(const JState &js, const int *tgt, int nt, const Plan &p,
                         const QueryOut &out, int cap, int fc, int *reset, const int *small,
-          hipStream_t st)
+                        hipStream_t st)
 {
     switch (p.tile * 8 + p.wpb) {
-        case 256 * 8 + 4: launch_shape<JL, EST, 256, 4>(js, tgt, nt, p, out, cap, fc, reset, small, st); break;
-        case 128 * 8 + 4: launch_shape<JL, EST, 128, 4>(js, tgt, nt, p, out, cap, fc, reset, small, st); break;
-        case 64 * 8 + 4: launch_shape<JL, EST, 64, 4>(js, tgt, nt, p, out, cap, fc, reset, small, st); break;
-        case 128 * 8 + 2: launch_shape<JL, EST, 128, 2>(js, tgt, nt, p, out, cap, fc, reset, small, st); break;
-        case 64 * 8 + 2: launch_shape<JL, EST, 64, 2>(js, tgt, nt, p, out, cap, fc, reset, small, st); break;
-        case 64 * 8 + 1: launch_shape<JL, EST, 64, 1>(js, tgt, nt, p, out, cap, fc, reset, small, st); break;
+        case 256 * 8 + 4:
+            launch_shape<JL, EST, 256, 4>(js, tgt, nt, p, out, cap, fc, reset, small, st);
+            break;
+        case 128 * 8 + 4:
+            launch_shape<JL, EST, 128, 4>(js, tgt, nt, p, out, cap, fc, reset, small, st);
+            break;
+        case 64 * 8 + 4:
+            launch_shape<JL, EST, 64, 4>(js, tgt, nt, p, out, cap, fc, reset, small, st);
+            break;
+        case 128 * 8 + 2:
+            launch_shape<JL, EST, 128, 2>(js, tgt, nt, p, out, cap, fc, reset, small, st);
+            break;
+        case 64 * 8 + 2:
+            launch_shape<JL, EST, 64, 2>(js, tgt, nt, p, out, cap, fc, reset, small, st);
+            break;
+        case 64 * 8 + 1:
+            launch_shape<JL, EST, 64, 1>(js, tgt, nt, p, out, cap, fc, reset, small, st);
+            break;
         case 1024 * 8 + 4:
             // one-shot tiles: every split within one tile (fold at 16 or 64 steps)
             if constexpr (JL >= 16) {
@@ -1621,8 +1644,7 @@ hipError_t launch_mode0(const JState &js, const int *tgt, int nt, const Plan &p,
 // tm: term mode; est: the spread estimate of checked precision (mode 0)
 template <int JL>
 hipError_t launch_jl(const JState &js, const int *tgt, int nt, const Plan &p, const QueryOut &out,
-                     int cap, int tm, bool est, int *reset, const int *small,
-          hipStream_t st)
+                     int cap, int tm, bool est, int *reset, const int *small, hipStream_t st)
 {
     // one workgroup per (target block, split) on a 1-D grid (xcd_place)
     if ((long long)p.grid_x * p.splits > 0x7fffffffLL) return hipErrorInvalidValue;
@@ -1645,17 +1667,17 @@ hipError_t launch_jl(const JState &js, const int *tgt, int nt, const Plan &p, co
     else if (tm == 0)
         return launch_mode0<JL, false>(js, tgt, nt, p, out, cap, fc, reset, small, st);
     else if (tm == 1)
-        hipLaunchKernelGGL((regf_kernel_jl<JL, 1, false, kTile, 4, JL == 4>), grid, dim3(kBlock), 0, st, js, tgt,
-                           nt, p.jspan, out, cap, fc, reset, p.grid_x, p.splits,
-                               target_arg<JL>(small, nt));
+        hipLaunchKernelGGL((regf_kernel_jl<JL, 1, false, kTile, 4, JL == 4>), grid,
+                           dim3(kBlock), 0, st, js, tgt, nt, p.jspan, out, cap, fc, reset,
+                           p.grid_x, p.splits, target_arg<JL>(small, nt));
     else if (tm == 2)
-        hipLaunchKernelGGL((regf_kernel_jl<JL, 2, false, kTile, 4, JL == 4>), grid, dim3(kBlock), 0, st, js, tgt,
-                           nt, p.jspan, out, cap, fc, reset, p.grid_x, p.splits,
-                               target_arg<JL>(small, nt));
+        hipLaunchKernelGGL((regf_kernel_jl<JL, 2, false, kTile, 4, JL == 4>), grid,
+                           dim3(kBlock), 0, st, js, tgt, nt, p.jspan, out, cap, fc, reset,
+                           p.grid_x, p.splits, target_arg<JL>(small, nt));
     else
-        hipLaunchKernelGGL((regf_kernel_jl<JL, 3, false, kTile, 4, JL == 4>), grid, dim3(kBlock), 0, st, js, tgt,
-                           nt, p.jspan, out, cap, fc, reset, p.grid_x, p.splits,
-                               target_arg<JL>(small, nt));
+        hipLaunchKernelGGL((regf_kernel_jl<JL, 3, false, kTile, 4, JL == 4>), grid,
+                           dim3(kBlock), 0, st, js, tgt, nt, p.jspan, out, cap, fc, reset,
+                           p.grid_x, p.splits, target_arg<JL>(small, nt));
     return hipGetLastError();
 }
 

@@ -39,7 +39,8 @@ StateView state_view(const double *base, int n)
 
 #pragma clang fp contract(off)
 __global__ __launch_bounds__(256) void predict_kernel(StateView st, int n, double t_new,
-                                                      double *__restrict__ jx, float *__restrict__ m32,
+                                                      double *__restrict__ jx,
+                                                      float *__restrict__ m32,
                                                       abyss::JRec *__restrict__ aos)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
