@@ -52,12 +52,12 @@ def same(a, b):
     return all(np.array_equal(p, q) for p, q in zip(a, b))
 
 
-@pytest.mark.parametrize("prec", [regf.PREC_SPLIT, regf.PREC_CHECKED])
-@pytest.mark.parametrize("n,nt", [(1024, 1), (1024, 64), (20000, 16), (20000, 300)])
+@pytest.mark.parametrize("n,nt,prec", [
+    (n, nt, p) for n, nt in ((1024, 1), (1024, 64), (20000, 16), (20000, 300))
+    for p in (regf.PREC_SPLIT, regf.PREC_CHECKED)])
 def test_replays_between_other_calls(n, nt, prec):
-    """One split and several, lists of up to 64 targets and longer ones."""
-    if prec == regf.PREC_CHECKED and nt > 256:
-        pytest.skip("allocates the checked pass's buffers inside the launch")
+    """One split and several, lists of up to 64 targets and longer ones (a
+    checked block of 300 with the count of its recomputation on the device)."""
     say(f"case: replay n={n} targets={nt} precision={prec}")
     js = [workloads.plummer_kroupa(n, seed=s, k_nb=30) for s in (1, 2)]
     rng = np.random.default_rng(n + nt)

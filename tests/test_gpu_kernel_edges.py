@@ -395,3 +395,34 @@ def test_regular_step_around_the_staged_lists(cap):
     for k in (0, 1, 2, 4):
         assert np.array_equal(out[0][k], out[1][k])
     assert np.array_equal(out[0][3][:, :700], out[1][3][:, :700]) and (out[0][2] > 0).all()
+
+
+@pytest.mark.parametrize("prec", [regf.PREC_SPLIT, regf.PREC_CHECKED])
+@pytest.mark.parametrize("n,cap,k_nb", [(4099, 64, 40), (4099, 20, 40), (32768, 64, 40)])
+def test_shapes_list_by_tile_alike(n, cap, k_nb, prec):
+    """Four lanes per target on a j-set of at most 32768 particles: every tile
+    and workgroup gives the bits of 256 j and 4 waves, with own targets in full
+    and partial tiles and overflowed lists."""
+    say(f"case: shapes by tile n={n} cap={cap} precision={prec}")
+    js = workloads.plummer_kroupa(n, seed=13, k_nb=k_nb)
+    rng = np.random.default_rng(n + cap)
+    t = np.concatenate([np.arange(n - 5, n), rng.permutation(n - 5)[:600]]).astype(np.int32)
+    with regf.Context(device=0, cap=cap, precision=prec) as c:
+        c.upload(js.m, js.x, js.v, js.r2)
+        for splits in (1, 3):
+            c.set_tuning(0, splits, 0, 4)
+            base = None
+            for tile, waves in [(256, 4), (128, 4), (64, 4), (128, 2), (64, 2), (64, 1)]:
+                c.set_shape(tile, waves)
+                got = [a.copy() for a in c.query(t)] + [c.last_recheck()]
+                p = c.plan()
+                assert (p["tile"], p["waves_per_block"], p["lanes_per_target"]) == (tile, waves, 4)
+                base = base or got
+                for a, b in zip(got, base):
+                    assert np.array_equal(a, b)
+            # and the lists are those of sixteen lanes, found a step at a time
+            c.set_shape()
+            c.set_tuning(0, splits, 0, 16)
+            want = c.query(t)
+            assert np.array_equal(base[2], want[2]) and np.array_equal(base[3], want[3])
+            assert (base[2] < 0).any() == (cap < k_nb)
