@@ -1093,12 +1093,12 @@ int ctx_launch_force(abyss_ctx_t c, bool to_host)
     if (c->n <= 0) return set_detail(c, ABYSS_ERR_NO_JSET, "no j-set uploaded");
     if (c->nt <= 0) return set_detail(c, ABYSS_ERR_INVALID_ARG, "no targets set");
     HIPCHK(c, hipSetDevice(c->device));
-    bool capturing = false;
-    {
+    if (!to_host) {   // a call that fetches has asked (refuse_capture)
+        bool capturing = false;
         int rc = ctx_capturing(c, &capturing);
         if (rc != ABYSS_OK) return rc;
+        if (capturing) c->captured = true;
     }
-    if (capturing) c->captured = true;
     // a recorded launch leaves its results in the device block, where a fetch
     // after a replay looks for them: no later launch may move that to the host
     if (c->captured) to_host = false;
