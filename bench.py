@@ -878,7 +878,7 @@ def bench_neighbour(args, reps=5):
         ms_d23 = (time.perf_counter() - t1) * 1e3
     out["irregular"] = {"targets": js.n, "list_entries": entries, "ms_per_call": ms_irr,
                         "entries_per_s": entries / (ms_irr * 1e-3),
-                        "includes": "target H2D, kernel, result D2H"}
+                        "includes": "target H2D, kernel writing mapped host memory, copies out"}
     out["regular_step"] = {"targets": js.n, "ms_per_call": ms_step, "query_ms_per_call": ms_query,
                            "correction_overhead_ms": ms_step - ms_query}
     out["update_radius"] = {"targets": js.n, "ms_per_call": ms_radius}

@@ -209,7 +209,16 @@ int abyss_ctx_query(abyss_ctx_t ctx, int nt, const int *targets, double *acc,
 
 /* Device-resident path: upload targets once, then enqueue any number of
  * launches on the context stream (no host synchronisation, results stay in
- * HBM), then fetch the last launch's results. */
+ * HBM), then fetch the last launch's results.
+ * A launch that does not wait (see the checked precision below) can be
+ * recorded into a HIP graph by a capture of abyss_ctx_stream and replayed
+ * after other targets of the same count have been set and other j-sets of the
+ * same size uploaded; fetch then returns what the replay computed.  It keeps
+ * the addresses of the context's buffers, which a larger block of targets, a
+ * larger j-set or a plan of more j-splits than the context has had replaces.
+ * A checked launch of 257 to 4096 targets allocates when it first runs, so it
+ * runs once before it is recorded.  Queries, regular steps, irregular forces
+ * and state updates fail with ABYSS_ERR_HIP under such a capture. */
 int abyss_ctx_set_targets(abyss_ctx_t ctx, int nt, const int *targets);
 int abyss_ctx_launch(abyss_ctx_t ctx);
 int abyss_ctx_sync(abyss_ctx_t ctx);
